@@ -515,6 +515,25 @@ __device__ inline int centre_out_row(int k, int h) {
   return above > below ? c + (k - m) : c - (k - m);
 }
 
+// Pixel of `lane` within its wave's ray tile of (1 << sh) x (64 >> sh) rays.
+// Lanes run through the tile in Z order, so that each four consecutive lanes
+// hold a 2 x 2 block of pixels: the vector-memory unit takes a wave's gather
+// four lanes at a time, and a 2 x 2 block's samples share cache lines more
+// often than four pixels of a row (16 lit 2D-TF views of 1920x1080 over a
+// 1 GiB volume: 30.0 -> 27.4 ms a launch; the 1D marches are bound
+// elsewhere and run as before).  The bits beyond the narrower edge go to the
+// longer one.
+__device__ inline void tile_pixel(int lane, int sh, int& x, int& y) {
+  const int m = min(sh, 6 - sh);  // bits of the tile's narrower edge
+  x = (lane & 1) | ((lane >> 1) & 2) | ((lane >> 2) & 4);
+  y = ((lane >> 1) & 1) | ((lane >> 2) & 2) | ((lane >> 3) & 4);
+  if (sh != 3) {
+    const int low = (1 << m) - 1, rest = lane >> (2 * m);
+    x = (x & low) | (sh > 3 ? rest << m : 0);
+    y = (y & low) | (sh < 3 ? rest << m : 0);
+  }
+}
+
 // A lane's pixel and ray: origin o, unit direction d (LOD-0 voxel space),
 // 1/d per axis (inf on axis-parallel rays) and the interval [t0, t1] inside
 // the volume box after the clip plane; hit false when the ray misses it.
@@ -540,8 +559,9 @@ __device__ inline bool setup_ray(const RaycastParams& P, int tile, int lane, Ray
   }
   const int tx = P.rect_x0 + tile % P.rect_w, ty = P.rect_y0 + centre_out_row(tile / P.rect_w, P.rect_h);
   const int sh = P.tile_shift;
-  const int px = (tx << sh) + (lane & ((1 << sh) - 1));
-  const int py = ty * (64 >> sh) + (lane >> sh);
+  int lx, ly;
+  tile_pixel(lane, sh, lx, ly);
+  const int px = (tx << sh) + lx, py = ty * (64 >> sh) + ly;
   if (px >= P.width || py >= P.height) return false;
   r.px = px;
   r.py = py;
@@ -1239,8 +1259,9 @@ __device__ inline void render_tile_staged(const RaycastParams& P, const float4* 
   }
   const int tx = P.rect_x0 + tile % P.rect_w, ty = P.rect_y0 + centre_out_row(tile / P.rect_w, P.rect_h);
   const int sh = P.tile_shift;
-  const int px = (tx << sh) + (lane & ((1 << sh) - 1));
-  const int py = ty * (64 >> sh) + (lane >> sh);
+  int lx, ly;
+  tile_pixel(lane, sh, lx, ly);
+  const int px = (tx << sh) + lx, py = ty * (64 >> sh) + ly;
   // every lane stays in the rounds (the staging needs all 64); lanes off
   // the image only help load
   const bool on_image = px < P.width && py < P.height;
