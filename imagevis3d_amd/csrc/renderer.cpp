@@ -1102,9 +1102,12 @@ int HipRenderer::upload_tf() {
     }
     if (t.dirty1d) {
       const size_t n = t.tf1d.size() / 4;
-      if (t.tf1d_dev.bytes < n * 16) TVK_HIP(t.tf1d_dev.alloc(n * 16));
+      if (t.tf1d_dev.bytes < (n + 1) * 16) TVK_HIP(t.tf1d_dev.alloc((n + 1) * 16));
       if (t.prefix1d_dev.bytes < (n + 1) * 4) TVK_HIP(t.prefix1d_dev.alloc((n + 1) * 4));
       TVK_HIP(hipMemcpyAsync(t.tf1d_dev.p, t.tf1d.data(), n * 16, hipMemcpyHostToDevice, stream_));
+      // the last entry again: entry i + 1 of a lookup is there for every i
+      TVK_HIP(hipMemcpyAsync(t.tf1d_dev.as<uint8_t>() + n * 16, t.tf1d.data() + (n - 1) * 4, 16,
+                             hipMemcpyHostToDevice, stream_));
       TVK_HIP(hipMemcpyAsync(t.prefix1d_dev.p, t.prefix1d.data(), (n + 1) * 4, hipMemcpyHostToDevice,
                              stream_));
       t.dirty1d = false;
@@ -2077,7 +2080,7 @@ bool HipRenderer::launch_ready_without_alloc(const tvk_view* views, uint32_t n, 
   for (const TfSet& t : tfs_) {
     if (t.dirty1d) {
       const size_t m = t.tf1d.size() / 4;
-      if (t.tf1d_dev.bytes < m * 16 || t.prefix1d_dev.bytes < (m + 1) * 4) return false;
+      if (t.tf1d_dev.bytes < (m + 1) * 16 || t.prefix1d_dev.bytes < (m + 1) * 4) return false;
     }
     if (t.dirty2d) {
       const size_t W = t.w2d, H = t.h2d;
