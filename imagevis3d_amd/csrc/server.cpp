@@ -487,6 +487,12 @@ void RenderServer::loop() {
     } else if (busy) {
       // lanes in flight: poll their events at a short interval
       cv_work_.wait_for(lk, std::chrono::microseconds(50));
+    } else if (!pending_.empty() && !stop_) {
+      // no lane in flight and nothing launched: the output memory is held
+      // by finished requests not collected yet.  The wait gives mu_ up, so
+      // that Wait can free it (a wait on "something is pending" would
+      // return at once, lock in hand, for ever)
+      cv_work_.wait_for(lk, std::chrono::milliseconds(1));
     } else {
       cv_work_.wait(lk, [&] { return stop_ || !pending_.empty(); });
     }

@@ -132,6 +132,32 @@ def test_admission_waits_for_output_memory():
     vols[0][0].cleanup()
 
 
+def test_submit_while_idle_lanes_wait_for_output_memory():
+    """Finished images nobody has collected hold all output memory, no lane
+    is in flight and a request is pending: the server must still take
+    further submits and go on once images are collected."""
+    import time
+    vols = make_volumes()[:1]
+    print("case serving submit with idle lanes and a full 1 MiB arena", flush=True)
+    srv = RenderServer(arena_bytes=1 << 20, lanes=4)
+    vid = srv.addVolume(vols[0][0])
+    view = dict(view_pos=(0.3, 0.4, 1.8), view_dir=(-0.3, -0.4, -1.8), fov=45.0, width=256,
+                height=256, tf_slot=0)
+    tickets = [srv.submit(vid, view) for _ in range(4)]
+    deadline = time.time() + 20.0
+    while srv.stats().completed < 4 and time.time() < deadline:
+        time.sleep(0.01)
+    assert srv.stats().completed == 4
+    tickets.append(srv.submit(vid, view))  # pending: its output memory is held
+    time.sleep(0.1)
+    tickets.append(srv.submit(vid, view))
+    out = [srv.wait(t, 20000) for t in tickets]
+    assert all(np.array_equal(o[0], out[0][0]) for o in out)
+    assert srv.stats().completed == 6
+    srv.close()
+    vols[0][0].cleanup()
+
+
 def test_paged_volumes_served_and_admitted_by_pool_memory():
     """Two paged volumes and an in-core one behind one server.  The GPU
     budget leaves the pool room for one paged batch's working set but not
