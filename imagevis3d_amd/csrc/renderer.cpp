@@ -660,7 +660,7 @@ int HipRenderer::resolve_check() {
   const double est = std::sqrt((double)(check_k_ - 1) * (double)*check_sse_h_ / (3.0 * px));
   check_stats_ = tvk_region_check{};
   check_stats_.rmse_estimate = (float)est;
-  check_stats_.check_samples = check_slot_.counters_h[kQueues];
+  check_stats_.check_samples = check_slot_.counters_h[kCounterBase];
   if (est > (double)check_max_) {
     if (int e = launch_jobs(check_slot_, &check_params_, 1, launch_info(check_params_.n_tf), false)) return e;
     check_stats_.fell_back = 1;
@@ -1693,7 +1693,7 @@ int launch_job_table_at(JobTable* table_h, void* dev_table, unsigned long long* 
   fill_job_table(table_h, jobs, n, li_in, tile_group, xcd_split, dev_counters, &culled, &groups);
   LaunchInfo li = li_in;
   li.group = groups > 0 ? 1 : 0;
-  const int words = kQueues + kJobCounters * n;
+  const int words = kCounterBase + kJobCounters * n;
   const size_t table_bytes = offsetof(JobTable, jobs) + (size_t)n * sizeof(RaycastParams);
   TVK_HIP(hipEventRecord(ev[0], stream_));
   TVK_HIP(hipMemcpyAsync(dev_table, table_h, table_bytes, hipMemcpyHostToDevice, stream_));
@@ -2057,9 +2057,9 @@ int HipRenderer::RenderBatch(const tvk_view* views, uint32_t n, tvk_view_stats* 
     for (int k = 0; k < cnt; ++k) {
       const uint32_t i = first + k;
       if (stats) {
-        stats[i].evaluated_samples = batch_slot_.counters_h[kQueues + kJobCounters * k];
-        stats[i].nominal_samples = batch_slot_.counters_h[kQueues + kJobCounters * k + 1];
-        stats[i].gathered_samples = batch_slot_.counters_h[kQueues + kJobCounters * k + 2];
+        stats[i].evaluated_samples = batch_slot_.counters_h[kCounterBase + kJobCounters * k];
+        stats[i].nominal_samples = batch_slot_.counters_h[kCounterBase + kJobCounters * k + 1];
+        stats[i].gathered_samples = batch_slot_.counters_h[kCounterBase + kJobCounters * k + 2];
         stats[i].lod = (uint32_t)lod;
         stats[i].reserved = 0;
       }
@@ -2138,9 +2138,9 @@ int HipRenderer::RenderBatchNoAlloc(const tvk_view* views, uint32_t n, void* con
   if (stats) {
     TVK_HIP(hipEventSynchronize(batch_slot_.ev[3]));
     for (uint32_t k = 0; k < n; ++k) {
-      stats[k].evaluated_samples = batch_slot_.counters_h[kQueues + kJobCounters * k];
-      stats[k].nominal_samples = batch_slot_.counters_h[kQueues + kJobCounters * k + 1];
-      stats[k].gathered_samples = batch_slot_.counters_h[kQueues + kJobCounters * k + 2];
+      stats[k].evaluated_samples = batch_slot_.counters_h[kCounterBase + kJobCounters * k];
+      stats[k].nominal_samples = batch_slot_.counters_h[kCounterBase + kJobCounters * k + 1];
+      stats[k].gathered_samples = batch_slot_.counters_h[kCounterBase + kJobCounters * k + 2];
       stats[k].lod = (uint32_t)lo;
       stats[k].reserved = 0;
     }
@@ -2305,8 +2305,8 @@ int HipRenderer::FrameStats(tvk_frame_stats* out) {
     TVK_HIP(hipEventElapsedTime(&all, sl.ev[0], sl.ev[3]));
     stats_.kernel_ms = k;
     stats_.paint_ms = all;
-    stats_.evaluated_samples = sl.counters_h[kQueues];
-    stats_.nominal_samples = sl.counters_h[kQueues + 1];
+    stats_.evaluated_samples = sl.counters_h[kCounterBase];
+    stats_.nominal_samples = sl.counters_h[kCounterBase + 1];
     stats_pending_ = false;
   }
   *out = stats_;

@@ -299,8 +299,8 @@ bool RenderServer::retire_locked() {
       Request& r = reqs_[L.tickets[k]];
       ++r.parts_retired;
       if (e == hipSuccess) {
-        const uint64_t nominal = L.cur->counters_h[kQueues + kJobCounters * k + 1];
-        r.evaluated += L.cur->counters_h[kQueues + kJobCounters * k];
+        const uint64_t nominal = L.cur->counters_h[kCounterBase + kJobCounters * k + 1];
+        r.evaluated += L.cur->counters_h[kCounterBase + kJobCounters * k];
         r.nominal += nominal;
         stats_.nominal_samples += nominal;
       } else if (r.status == TVK_OK) {

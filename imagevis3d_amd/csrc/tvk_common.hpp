@@ -193,6 +193,11 @@ constexpr int kGroupMax = 4;
 // form one index space that the persistent kernel's waves drain.
 constexpr int kMaxJobs = 64;
 constexpr int kQueues = 8;  // one tile queue per XCD
+// The queue heads lie a memory channel apart: device-scope atomics are done
+// at the memory side, and on one line they are served one by one (about 75
+// per us for the whole chip, all eight queues together).
+constexpr int kQueueStride = 32;               // u64 words from one head to the next
+constexpr int kCounterBase = kQueues * kQueueStride;  // first word of the jobs' counters
 struct JobTableHeader {
   int32_t n_jobs;
   int32_t total_tiles;
@@ -201,8 +206,9 @@ struct JobTableHeader {
   int32_t n_tf_lds;     // > 0: every job reads this 1D TF, staged into LDS
   int32_t pad_[3];
   const float* tf_lds;
-  // [0, 8) per-XCD tile queue heads, then per job j: [8 + 3j] evaluated
-  // samples, [9 + 3j] nominal samples, [10 + 3j] gathered samples (those
+  // per-XCD tile queue heads every kQueueStride words, then from
+  // b = kCounterBase per job j: [b + 3j] evaluated samples, [b + 3j + 1]
+  // nominal samples, [b + 3j + 2] gathered samples (those
   // whose voxels the march loaded: a TF group's walk is counted on its
   // leader and 0 on its members; a job marched alone gathers the samples
   // it evaluates)
@@ -216,7 +222,7 @@ struct JobTable {
   RaycastParams jobs[kMaxJobs];
 };
 constexpr int kJobCounters = 3;
-constexpr int kCounterWords = kQueues + kJobCounters * kMaxJobs;
+constexpr int kCounterWords = kCounterBase + kJobCounters * kMaxJobs;
 
 // One brick to cut out of a flat level into a pool slot.
 struct BrickJob {
