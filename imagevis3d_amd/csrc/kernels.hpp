@@ -81,11 +81,13 @@ hipError_t launch_region_detail(const void* const* levels, const int64_t (*dims)
 hipError_t launch_fill_u64(unsigned long long* p, int64_t n, unsigned long long v,
                            hipStream_t stream);
 
-// Empty flags (u8) of n_cells empty-space cells for one TF (mode 0/1: TF
-// prefix counts over n_tf entries or columns; mode 2: iso value).
-hipError_t launch_cell_empty(const uint32_t* cell_range, int64_t n_cells, const int32_t* prefix,
-                             int n_tf, float tf_scale, int mode, float iso_value, uint8_t* out,
-                             hipStream_t stream);
+// Codes (u8: bit 0 empty, above it the block level) of all levels' cells for
+// one TF (mode 0/1: TF prefix counts over n_tf entries or columns; mode 2:
+// iso value).  lods_dev: lods[0..n_lod) on the device; per_brick: cells
+// along a brick.
+hipError_t launch_cell_codes(const LodInfo* lods_dev, const LodInfo* lods, int n_lod, int per_brick,
+                             const uint32_t* cell_range, const int32_t* prefix, int n_tf, float tf_scale,
+                             int mode, float iso_value, uint8_t* out, hipStream_t stream);
 
 // Device-side synthetic volumes (TVK_VOL_FBM_PLANES, _NOISE_TUBES,
 // _FBM_SPHERES): z slab [z0, z0 + nz) of a dims volume into `out`.

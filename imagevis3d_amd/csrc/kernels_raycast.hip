@@ -652,6 +652,64 @@ __device__ inline bool setup_ray(const RaycastParams& P, int tile, int lane, Ray
   return true;
 }
 
+// The walk of one ray over the march units of its level: the empty-space
+// cells (P.cell voxels) when skipping, else the bricks.
+struct Walk {
+  float od[3], oo[3];  // the ray in level voxels
+  float ul0[3];        // unit edge in LOD-0 voxels
+  float invU;
+  int ucount[3];       // units of the level
+  int per_brick;       // units along a brick
+};
+
+__device__ inline Walk make_walk(const RaycastParams& P, const LodInfo& lv, const float (&o)[3],
+                                 const float (&d)[3]) {
+  Walk w;
+  const int U = P.cell;
+  w.per_brick = P.brick / U;
+  w.invU = 1.f / (float)U;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    w.od[i] = d[i] * lv.to_level[i];
+    w.oo[i] = o[i] * lv.to_level[i];
+    w.ul0[i] = (float)U / lv.to_level[i];
+    w.ucount[i] = (lv.dims[i] + U - 1) / U;
+  }
+  return w;
+}
+
+// The unit c of the sample at ray parameter tk, and its brick's place b in
+// the level's grid.
+__device__ inline void unit_index(const Walk& w, float tk, int (&c)[3], int (&b)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    c[i] = (int)__builtin_amdgcn_fmed3f(fmaf(tk, w.od[i], w.oo[i]) * w.invU, 0.f, (float)(w.ucount[i] - 1));
+  if ((w.per_brick & (w.per_brick - 1)) == 0) {  // wave-uniform: a shift for the usual edges
+    const int sh = __builtin_ctz((unsigned)w.per_brick);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) b[i] = c[i] >> sh;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) b[i] = c[i] / w.per_brick;
+  }
+}
+
+// First sample past the aligned block of 2^level units (per axis) that holds
+// unit c, at least k + 1, at most n.
+__device__ inline int unit_end(const Walk& w, const float (&o)[3], const float (&d)[3], const float (&inv)[3],
+                               const int (&c)[3], int level, float t0, float step, int k, int n) {
+  float tb = kInf;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (d[i] != 0.f) {
+      const int at = c[i] >> level << level;
+      const float face = (float)(d[i] > 0.f ? at + (1 << level) : at) * w.ul0[i];
+      tb = fminf(tb, (face - o[i]) * inv[i]);
+    }
+  }
+  return min(max((int)ceilf((tb - t0) / step - 0.5f), k + 1), n);
+}
+
 template <typename T, bool LINEAR, int BATCH, int MODE, bool TF_LDS>
 __device__ inline void render_tile(const RaycastParams& P, const float4* __restrict__ tf4, int tile,
                                    int lane, uint32_t& n_eval, uint32_t& n_nom) {
@@ -685,20 +743,9 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
     const int n = (int)ceilf(L / step);
     const float lastlen = fmaxf(L - (float)(n - 1) * step, 0.f);
     const LodInfo& lv = P.level;
-    // The ray walks march units of P.cell level voxels: the empty-space
-    // cells when skipping (a cell lies inside one brick), else the bricks.
-    const int U = P.cell;
-    const int per_brick = P.brick / U;
-    const float invU = 1.f / (float)U;
-    float od[3], oo[3], ul0[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      od[i] = d[i] * lv.to_level[i];
-      oo[i] = o[i] * lv.to_level[i];
-      ul0[i] = (float)U / lv.to_level[i];  // unit edge in LOD-0 voxels
-    }
-    const int ucount[3] = {(lv.dims[0] + U - 1) / U, (lv.dims[1] + U - 1) / U,
-                           (lv.dims[2] + U - 1) / U};
+    const Walk walk = make_walk(P, lv, o, d);
+    const float(&od)[3] = walk.od;
+    const float(&oo)[3] = walk.oo;
     const float tfmax = (float)(P.n_tf - 1);
     const SlotGeo G = slot_geo(P.slot_edge);
     float Lh[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // light direction, half vector
@@ -735,30 +782,18 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
         if (k >= kend) {
           const float len0 = (k == n - 1) ? lastlen : step;
           const float tk = fmaf((float)k, step, t0) + 0.5f * len0;
-          int c[3];
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            c[i] = clampi((int)floorf(fmaf(tk, od[i], oo[i]) * invU), 0, ucount[i] - 1);
-          float tb = kInf;
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            if (d[i] != 0.f) {
-              const float face = (float)(d[i] > 0.f ? c[i] + 1 : c[i]) * ul0[i];
-              tb = fminf(tb, (face - o[i]) * inv[i]);
-            }
-          }
-          kend = min(max((int)ceilf((tb - t0) / step - 0.5f), k + 1), n);
-          int b[3];
-#pragma unroll
-          for (int i = 0; i < 3; ++i) b[i] = c[i] / per_brick;
+          int c[3], b[3];
+          unit_index(walk, tk, c, b);
           const int gid = lv.brick_base + (b[2] * lv.grid[1] + b[1]) * lv.grid[0] + b[0];
-          const uint8_t empty =
-              P.skip ? gload(P.cell_empty + (lv.cell_base + (c[2] * ucount[1] + c[1]) * ucount[0] + c[0])) : 0;
+          const uint32_t code =
+              P.skip ? gload(P.cell_code + (lv.cell_base + (c[2] * walk.ucount[1] + c[1]) * walk.ucount[0] + c[0])) : 0u;
+          const bool empty = code & 1u;
           base = brick_base<T>(P, gid);
           if (P.blend_bits < 32 && gid != blend_gid) {
             blend_round(P.blend_bits, C0, C1, C2, A);
             blend_gid = gid;
           }
+          kend = unit_end(walk, o, d, inv, c, (int)(code >> 1), t0, step, k, n);
           if (empty) {
             k = kend;
             continue;
@@ -862,29 +897,16 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
     while (k < n) {
       const float len0 = (k == n - 1) ? lastlen : step;
       const float tk = fmaf((float)k, step, t0) + 0.5f * len0;
-      int c[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        c[i] = clampi((int)floorf(fmaf(tk, od[i], oo[i]) * invU), 0, ucount[i] - 1);
-      float tb = kInf;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        if (d[i] != 0.f) {
-          const float face = (float)(d[i] > 0.f ? c[i] + 1 : c[i]) * ul0[i];
-          tb = fminf(tb, (face - o[i]) * inv[i]);
-        }
-      }
-      int kend = (int)ceilf((tb - t0) / step - 0.5f);
-      kend = min(max(kend, k + 1), n);
-      int b[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) b[i] = c[i] / per_brick;
+      int c[3], b[3];
+      unit_index(walk, tk, c, b);
       const int gid = lv.brick_base + (b[2] * lv.grid[1] + b[1]) * lv.grid[0] + b[0];
-      // the cell's empty flag and the brick's slot are independent loads
-      const uint8_t empty =
+      // the cell's code and the brick's slot are independent loads
+      const uint32_t code =
           (MODE != kModeMIP && P.skip)
-              ? gload(P.cell_empty + (lv.cell_base + (c[2] * ucount[1] + c[1]) * ucount[0] + c[0]))
-              : 0;
+              ? gload(P.cell_code + (lv.cell_base + (c[2] * walk.ucount[1] + c[1]) * walk.ucount[0] + c[0]))
+              : 0u;
+      const bool empty = code & 1u;
+      const int kend = unit_end(walk, o, d, inv, c, (int)(code >> 1), t0, step, k, n);
       const T* __restrict__ base = brick_base<T>(P, gid);
       if (kBlends && P.blend_bits < 32 && gid != blend_gid) {
         blend_round(P.blend_bits, C0, C1, C2, A);
@@ -1037,35 +1059,28 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
 // that some member needs.  Returns whether the unit has samples to gather.
 template <typename T, bool LINEAR>
 __device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* const (&Q)[kGroupMax], int F,
-                                  const Ray& r, const float (&od)[3], const float (&oo)[3],
-                                  const float (&ul0)[3], const int (&ucount)[3], float invU, int per_brick,
+                                  const Ray& r, const Walk& walk,
                                   int k, int n, float t0, float step, float lastlen, uint32_t live, int& kend,
                                   uint32_t& need, const T* __restrict__& base, float (&g0)[3], int& blend_gid,
                                   float (&C)[kGroupMax][3], float (&A)[kGroupMax]) {
   const LodInfo& lv = P.level;
   const float len0 = (k == n - 1) ? lastlen : step;
   const float tk = fmaf((float)k, step, t0) + 0.5f * len0;
-  int c[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) c[i] = clampi((int)floorf(fmaf(tk, od[i], oo[i]) * invU), 0, ucount[i] - 1);
-  float tb = kInf;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    if (r.d[i] != 0.f) {
-      const float face = (float)(r.d[i] > 0.f ? c[i] + 1 : c[i]) * ul0[i];
-      tb = fminf(tb, (face - r.o[i]) * r.inv[i]);
-    }
-  }
-  kend = min(max((int)ceilf((tb - t0) / step - 0.5f), k + 1), n);
-  int b[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) b[i] = c[i] / per_brick;
+  int c[3], b[3];
+  unit_index(walk, tk, c, b);
   const int gid = lv.brick_base + (b[2] * lv.grid[1] + b[1]) * lv.grid[0] + b[0];
-  const int64_t cidx = lv.cell_base + (c[2] * ucount[1] + c[1]) * ucount[0] + c[0];
+  const int64_t cidx = lv.cell_base + (c[2] * walk.ucount[1] + c[1]) * walk.ucount[0] + c[0];
+  // each live member's code; the unit is the block uniform for all of them
   need = 0;
+  uint32_t level = P.skip ? 15u : 0u;
 #pragma unroll
   for (int f = 0; f < kGroupMax; ++f)
-    if (f < F && (live >> f & 1u) && !(P.skip && gload(Q[f]->cell_empty + cidx))) need |= 1u << f;
+    if (f < F && (live >> f & 1u)) {
+      const uint32_t code = P.skip ? gload(Q[f]->cell_code + cidx) : 0u;
+      if (!(code & 1u)) need |= 1u << f;
+      level = min(level, code >> 1);
+    }
+  kend = unit_end(walk, r.o, r.d, r.inv, c, (int)level, t0, step, k, n);
   base = brick_base<T>(P, gid);
   if (P.blend_bits < 32 && gid != blend_gid) {
 #pragma unroll
@@ -1080,7 +1095,7 @@ __device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* c
   }
   if (P.touch) P.touch[gid] = P.frame;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) g0[i] = oo[i] - (float)(b[i] * P.brick - P.apron) - (LINEAR ? 0.5f : 0.f);
+  for (int i = 0; i < 3; ++i) g0[i] = walk.oo[i] - (float)(b[i] * P.brick - P.apron) - (LINEAR ? 0.5f : 0.f);
   return true;
 }
 
@@ -1116,18 +1131,8 @@ __device__ inline void render_tile_group(const JobTable* __restrict__ tab, const
     const int n = (int)ceilf(L / step);
     const float lastlen = fmaxf(L - (float)(n - 1) * step, 0.f);
     const LodInfo& lv = P.level;
-    const int U = P.cell;
-    const int per_brick = P.brick / U;
-    const float invU = 1.f / (float)U;
-    float od[3], oo[3], ul0[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      od[i] = r.d[i] * lv.to_level[i];
-      oo[i] = r.o[i] * lv.to_level[i];
-      ul0[i] = (float)U / lv.to_level[i];
-    }
-    const int ucount[3] = {(lv.dims[0] + U - 1) / U, (lv.dims[1] + U - 1) / U,
-                           (lv.dims[2] + U - 1) / U};
+    const Walk walk = make_walk(P, lv, r.o, r.d);
+    const float(&od)[3] = walk.od;
     const SlotGeo G = slot_geo(P.slot_edge);
     float Lh[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // light direction, half vector
     {
@@ -1149,8 +1154,7 @@ __device__ inline void render_tile_group(const JobTable* __restrict__ tab, const
     float g0[3] = {0.f, 0.f, 0.f};
     const T* __restrict__ base = nullptr;
     while (k < n) {
-      if (k >= kend && !group_unit<T, LINEAR>(P, Q, F, r, od, oo, ul0, ucount, invU, per_brick, k, n, t0, step,
-                                              lastlen, live, kend, need, base, g0, blend_gid, C, A)) {
+      if (k >= kend && !group_unit<T, LINEAR>(P, Q, F, r, walk, k, n, t0, step, lastlen, live, kend, need, base, g0, blend_gid, C, A)) {
         k = kend;
         continue;
       }
@@ -1348,17 +1352,9 @@ __device__ inline void render_tile_staged(const RaycastParams& P, const float4* 
   const int n = (hit && L > 0.f) ? (int)ceilf(L / step) : 0;
   const float lastlen = fmaxf(L - (float)(n - 1) * step, 0.f);
   const LodInfo& lv = P.level;
-  const int U = P.cell;
-  const int per_brick = P.brick / U;
-  const float invU = 1.f / (float)U;
-  float od[3], oo[3], ul0[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    od[i] = d[i] * lv.to_level[i];
-    oo[i] = o[i] * lv.to_level[i];
-    ul0[i] = (float)U / lv.to_level[i];
-  }
-  const int ucount[3] = {(lv.dims[0] + U - 1) / U, (lv.dims[1] + U - 1) / U, (lv.dims[2] + U - 1) / U};
+  const Walk walk = make_walk(P, lv, o, d);
+  const float(&od)[3] = walk.od;
+  const float(&oo)[3] = walk.oo;
   const float tfmax = (float)(P.n_tf - 1);
   const SlotGeo G = slot_geo(P.slot_edge);
   const int Smax = G.S - 2;
@@ -1377,25 +1373,13 @@ __device__ inline void render_tile_staged(const RaycastParams& P, const float4* 
         }
         const float len0 = (k == n - 1) ? lastlen : step;
         const float tk = fmaf((float)k, step, t0) + 0.5f * len0;
-        int c[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          c[i] = clampi((int)floorf(fmaf(tk, od[i], oo[i]) * invU), 0, ucount[i] - 1);
-        float tb = kInf;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          if (d[i] != 0.f) {
-            const float face = (float)(d[i] > 0.f ? c[i] + 1 : c[i]) * ul0[i];
-            tb = fminf(tb, (face - o[i]) * inv[i]);
-          }
-        }
-        kend = min(max((int)ceilf((tb - t0) / step - 0.5f), k + 1), n);
-        int b[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) b[i] = c[i] / per_brick;
+        int c[3], b[3];
+        unit_index(walk, tk, c, b);
         gid = lv.brick_base + (b[2] * lv.grid[1] + b[1]) * lv.grid[0] + b[0];
-        const uint8_t empty =
-            P.skip ? gload(P.cell_empty + (lv.cell_base + (c[2] * ucount[1] + c[1]) * ucount[0] + c[0])) : 0;
+        const uint32_t code =
+            P.skip ? gload(P.cell_code + (lv.cell_base + (c[2] * walk.ucount[1] + c[1]) * walk.ucount[0] + c[0])) : 0u;
+        const bool empty = code & 1u;
+        kend = unit_end(walk, o, d, inv, c, (int)(code >> 1), t0, step, k, n);
         base = brick_base<T>(P, gid);
         if (P.blend_bits < 32 && gid != blend_gid) {
           blend_round(P.blend_bits, C0, C1, C2, A);
@@ -1503,26 +1487,94 @@ __device__ inline void render_tile_staged(const RaycastParams& P, const float4* 
   if (on_image) gstore(P.framebuffer + ((int64_t)py * P.width + px), over_background(P, py, C0, C1, C2, A));
 }
 
-// Empty flag per empty-space cell for one TF: the TF entries (1D) or
-// columns (2D) that the cell's value range reaches hold no alpha > 0, or
-// (isosurface) the cell's maximum is below the iso value.  Such cells
-// contribute nothing to any ray, so the raycast skips them.
-__global__ void cell_empty_kernel(const uint32_t* __restrict__ cell_range, int64_t n_cells,
-                                  const int32_t* __restrict__ prefix, int n_tf, float tf_scale,
-                                  int mode, float iso_value, uint8_t* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_cells) return;
-  const uint32_t r = cell_range[i];
-  bool empty;
-  if (mode == kModeIso) {
-    empty = (float)(r >> 16) < iso_value;
-  } else {
-    const float tfmax = (float)(n_tf - 1);
-    const int i0 = (int)clampf((float)(r & 0xffffu) * tf_scale, 0.f, tfmax);
-    const int i1 = min((int)clampf((float)(r >> 16) * tf_scale, 0.f, tfmax) + 1, n_tf - 1);
-    empty = prefix[i1 + 1] - prefix[i0] == 0;
+// Code per empty-space cell for one TF.  Bit 0: empty -- the TF entries (1D)
+// or columns (2D) that the cell's value range reaches hold no alpha > 0, or
+// (isosurface) the cell's maximum is below the iso value; such cells
+// contribute nothing to any ray, so the raycast skips them.  The bits above:
+// the largest level such that the aligned block of 2^level cells per axis
+// that holds the cell is all empty or all not, and inside one brick; a ray
+// crosses it as one march unit.  With one unit per cell of 16 voxels, the
+// walk through 512^3 with hardly an empty cell was a quarter of the march: a
+// 1080p frame of it 1.12 -> 0.83 ms, 8 views of a 301 x 257 x 193 scan with
+// readback 1.65 -> 1.49 ms, 16 lit 2D-TF views of 1 GiB 27.4 -> 24.6 ms.
+//
+// A work-group takes an aligned region of 16^3 cells of one level, cells in
+// Z order: a wave's 64 lanes hold a block of 4^3 and its bytes blocks of
+// 2^3, so levels 1 and 2 come from the wave's ballots, and levels 3 and 4
+// from the 64 blocks' states in LDS.  Cells beyond the level agree with any
+// block.  Bound by the reads of the ranges, 4 B per cell.
+constexpr int kCodeEdge = 16;  // cells along a work-group's region
+
+__global__ __launch_bounds__(256) void cell_code_kernel(const LodInfo* __restrict__ lods, int n_lod, int max_level,
+                                                        const uint32_t* __restrict__ cell_range,
+                                                        const int32_t* __restrict__ prefix, int n_tf,
+                                                        float tf_scale, int mode, float iso_value,
+                                                        uint8_t* __restrict__ out) {
+  __shared__ uint32_t s_state[64];  // per 4^3 block: bit 0 all empty, bit 1 all not
+  // this work-group's level and region (uniform)
+  int l = 0, r = (int)blockIdx.x, rx = 0, ry = 0;
+  for (; l < n_lod; ++l) {
+    rx = (lods[l].cells[0] + kCodeEdge - 1) / kCodeEdge;
+    ry = (lods[l].cells[1] + kCodeEdge - 1) / kCodeEdge;
+    const int rz = (lods[l].cells[2] + kCodeEdge - 1) / kCodeEdge;
+    if (r < rx * ry * rz) break;
+    r -= rx * ry * rz;
   }
-  out[i] = empty ? 1 : 0;
+  if (l == n_lod) return;
+  const LodInfo& lv = lods[l];
+  const int x0 = r % rx * kCodeEdge, y0 = r / rx % ry * kCodeEdge, z0 = r / (rx * ry) * kCodeEdge;
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const float tfmax = (float)(n_tf - 1);
+  constexpr int kPer = kCodeEdge * kCodeEdge * kCodeEdge / 256;
+  uint32_t codes[kPer];
+#pragma unroll
+  for (int it = 0; it < kPer; ++it) {
+    const int m = it * 256 + tid;
+    const int x = x0 + ((m & 1) | (m >> 2 & 2) | (m >> 4 & 4) | (m >> 6 & 8));
+    const int y = y0 + ((m >> 1 & 1) | (m >> 3 & 2) | (m >> 5 & 4) | (m >> 7 & 8));
+    const int z = z0 + ((m >> 2 & 1) | (m >> 4 & 2) | (m >> 6 & 4) | (m >> 8 & 8));
+    const bool in = x < lv.cells[0] && y < lv.cells[1] && z < lv.cells[2];
+    bool empty = false;
+    if (in) {
+      const uint32_t v = cell_range[lv.cell_base + ((int64_t)z * lv.cells[1] + y) * lv.cells[0] + x];
+      if (mode == kModeIso) {
+        empty = (float)(v >> 16) < iso_value;
+      } else {
+        const int i0 = (int)clampf((float)(v & 0xffffu) * tf_scale, 0.f, tfmax);
+        const int i1 = min((int)clampf((float)(v >> 16) * tf_scale, 0.f, tfmax) + 1, n_tf - 1);
+        empty = prefix[i1 + 1] - prefix[i0] == 0;
+      }
+    }
+    const unsigned long long all = __ballot(empty || !in), none = __ballot(!empty);
+    const unsigned long long same = empty ? all : none;
+    const uint32_t byte = (uint32_t)(same >> (lane & ~7)) & 0xffu;
+    codes[it] = (in ? 0u : 0x80u) | (empty ? 1u : 0u) | (same == ~0ull ? 4u : (byte == 0xffu ? 2u : 0u));
+    if (lane == 0) s_state[m >> 6] = (all == ~0ull ? 1u : 0u) | (none == ~0ull ? 2u : 0u);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kPer; ++it) {
+    const int m = it * 256 + tid;
+    uint32_t code = codes[it];
+    if (code & 0x80u) continue;
+    const uint32_t want = (code & 1u) ? 1u : 2u;
+    uint32_t level = code >> 1;
+    if (level == 2u) {  // the 8 blocks of 8^3 cells around this one, then all 64
+      const int at = m >> 6;
+      uint32_t st = 3u;
+      for (int j = 0; j < 8; ++j) st &= s_state[(at & ~7) + j];
+      if (st & want) {
+        level = 3u;
+        for (int j = 0; j < 64; ++j) st &= s_state[j];
+        if (st & want) level = 4u;
+      }
+    }
+    const int x = x0 + ((m & 1) | (m >> 2 & 2) | (m >> 4 & 4) | (m >> 6 & 8));
+    const int y = y0 + ((m >> 1 & 1) | (m >> 3 & 2) | (m >> 5 & 4) | (m >> 7 & 8));
+    const int z = z0 + ((m >> 2 & 1) | (m >> 4 & 2) | (m >> 6 & 4) | (m >> 8 & 8));
+    out[lv.cell_base + ((int64_t)z * lv.cells[1] + y) * lv.cells[0] + x] =
+        (uint8_t)((code & 1u) | min(level, (uint32_t)max_level) << 1);
+  }
 }
 
 // Background of every pixel outside its job's tile rect (such rays miss the
@@ -1617,17 +1669,8 @@ __device__ inline void render_tile_group_runs(const JobTable* __restrict__ tab, 
   const int n = (mine && r.hit && L > 0.f) ? (int)ceilf(L / step) : 0;
   const float lastlen = n > 0 ? fmaxf(L - (float)(n - 1) * step, 0.f) : 0.f;
   const LodInfo& lv = P.level;
-  const int U = P.cell;
-  const int per_brick = P.brick / U;
-  const float invU = 1.f / (float)U;
-  float od[3], oo[3], ul0[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    od[i] = r.d[i] * lv.to_level[i];
-    oo[i] = r.o[i] * lv.to_level[i];
-    ul0[i] = (float)U / lv.to_level[i];
-  }
-  const int ucount[3] = {(lv.dims[0] + U - 1) / U, (lv.dims[1] + U - 1) / U, (lv.dims[2] + U - 1) / U};
+  const Walk walk = make_walk(P, lv, r.o, r.d);
+  const float(&od)[3] = walk.od;
   const SlotGeo G = slot_geo(P.slot_edge);
   uint32_t live = n > 0 ? (1u << F) - 1 : 0u;  // members still compositing
   uint32_t need = 0;                           // live members whose TF keeps the current unit
@@ -1642,7 +1685,7 @@ __device__ inline void render_tile_group_runs(const JobTable* __restrict__ tab, 
         ready = true;
         break;
       }
-      if (!group_unit<T, LINEAR>(P, Q, F, r, od, oo, ul0, ucount, invU, per_brick, k, n, t0, step, lastlen, live,
+      if (!group_unit<T, LINEAR>(P, Q, F, r, walk, k, n, t0, step, lastlen, live,
                                  kend, need, base, g0, blend_gid, C, A))
         k = kend;
     }
@@ -1970,13 +2013,20 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
 
 }  // namespace
 
-hipError_t launch_cell_empty(const uint32_t* cell_range, int64_t n_cells, const int32_t* prefix,
-                             int n_tf, float tf_scale, int mode, float iso_value, uint8_t* out,
-                             hipStream_t stream) {
-  if (n_cells <= 0) return hipSuccess;
-  const unsigned blocks = (unsigned)((n_cells + 255) / 256);
-  cell_empty_kernel<<<blocks, 256, 0, stream>>>(cell_range, n_cells, prefix, n_tf, tf_scale,
-                                                mode == 2 ? kModeIso : mode, iso_value, out);
+hipError_t launch_cell_codes(const LodInfo* lods_dev, const LodInfo* lods, int n_lod, int per_brick,
+                             const uint32_t* cell_range, const int32_t* prefix, int n_tf, float tf_scale,
+                             int mode, float iso_value, uint8_t* out, hipStream_t stream) {
+  int64_t regions = 0;
+  for (int l = 0; l < n_lod; ++l) {
+    int64_t r = 1;
+    for (int i = 0; i < 3; ++i) r *= (lods[l].cells[i] + kCodeEdge - 1) / kCodeEdge;
+    regions += r;
+  }
+  if (regions <= 0) return hipSuccess;
+  // blocks that divide the brick lie inside one (16 cells at most)
+  const int max_level = std::min(4, __builtin_ctz((unsigned)per_brick));
+  cell_code_kernel<<<(unsigned)regions, 256, 0, stream>>>(lods_dev, n_lod, max_level, cell_range, prefix, n_tf,
+                                                          tf_scale, mode == 2 ? kModeIso : mode, iso_value, out);
   return hipGetLastError();
 }
 

@@ -1540,7 +1540,7 @@ void HipRenderer::build_params(RaycastParams* p, int lod, const CameraState& cam
   p->page_table = pool_.page_table.as<uint64_t>();
   p->brick_range = pool_.brick_range.as<float>();
   p->cell_range = cell_range_.as<uint32_t>();
-  p->cell_empty = tfs.cell_empty[mode_index()].as<uint8_t>();
+  p->cell_code = tfs.cell_code[mode_index()].as<uint8_t>();
   p->cell = skip_ ? cell_ : brick_;
   p->tf = tfs.tf1d_dev.as<float>();
   p->tf_prefix = tfs.prefix1d_dev.as<int32_t>();
@@ -1623,7 +1623,7 @@ static bool same_but_tf(const RaycastParams& a, const RaycastParams& b) {
     p->n_tf = 0;
     p->tf = nullptr;
     p->tf_prefix = nullptr;
-    p->cell_empty = nullptr;
+    p->cell_code = nullptr;
     p->framebuffer = nullptr;
     p->group_n = 0;
     memset(p->group_jobs, 0, sizeof p->group_jobs);
@@ -1789,13 +1789,13 @@ int HipRenderer::prepare_cells(int tf_slot, int mode) {
   for (const uint64_t v : {cells_gen_, (uint64_t)mode, t.version, (uint64_t)(mode == 2 ? iso_bits : 0),
                            (uint64_t)scale_bits, (uint64_t)n})
     key = (key ^ v) * 1099511628211ull;
-  DevBuf& flags = t.cell_empty[mode];
+  DevBuf& flags = t.cell_code[mode];
   if (key == t.cell_key[mode] && flags.p) return TVK_OK;
   if (flags.bytes < (size_t)total_cells_) TVK_HIP(flags.alloc((size_t)total_cells_));
   const int32_t* prefix_dev = mode == 1 ? t.prefix2d_dev.as<int32_t>() : t.prefix1d_dev.as<int32_t>();
   if (mode != 2 && (n < 1 || !prefix_dev)) return state_fail("TF not uploaded");
-  TVK_HIP(launch_cell_empty(cell_range_.as<uint32_t>(), total_cells_, prefix_dev, n, scale, mode,
-                            iso, flags.as<uint8_t>(), stream_));
+  TVK_HIP(launch_cell_codes(lods_dev_.as<LodInfo>(), lods_, n_lod_, brick_ / cell_, cell_range_.as<uint32_t>(),
+                            prefix_dev, n, scale, mode, iso, flags.as<uint8_t>(), stream_));
   t.cell_key[mode] = key;
   return TVK_OK;
 }
@@ -2089,7 +2089,7 @@ bool HipRenderer::launch_ready_without_alloc(const tvk_view* views, uint32_t n, 
   }
   if (skip_ && total_cells_ > 0)
     for (uint32_t i = 0; i < n; ++i)
-      if (tfs_[views[i].tf_slot].cell_empty[mode].bytes < (size_t)total_cells_) return false;
+      if (tfs_[views[i].tf_slot].cell_code[mode].bytes < (size_t)total_cells_) return false;
   return true;
 }
 
@@ -2360,7 +2360,7 @@ int HipRenderer::MemStats(tvk_mem_stats* out) {
   for (auto& l : levels_) a += l.bytes;
   for (const TfSet& t : tfs_) {
     a += t.tf1d_dev.bytes + t.prefix1d_dev.bytes + t.tf2d_dev.bytes + t.prefix2d_dev.bytes;
-    for (const DevBuf& f : t.cell_empty) a += f.bytes;
+    for (const DevBuf& f : t.cell_code) a += f.bytes;
   }
   for (const LaunchSlot* sl : {&paint_slots_[0], &paint_slots_[1], &batch_slot_})
     a += sl->table.bytes + sl->counters.bytes;

@@ -98,8 +98,8 @@ struct TfSet {
   DevBuf region_code;     // per LOD-0 region: chosen level | 0x80 when TF-empty
   DevBuf region_code0;    // the same with every region at level 0
   uint64_t region_key = 0;
-  DevBuf cell_empty[3];      // per render mode: u8 per empty-space cell of every level
-  uint64_t cell_key[3] = {};  // what each cell_empty was built for
+  DevBuf cell_code[3];       // per render mode: u8 per empty-space cell of every level
+  uint64_t cell_key[3] = {};  // what each cell_code was built for
 };
 
 // A camera (Tuvok's view position / direction / up, FoV or ortho extent).
@@ -279,7 +279,7 @@ class HipRenderer : public PoolClient {
   int RenderBatchNoAlloc(const tvk_view* views, uint32_t n, void* const* dev_rgba, tvk_view_stats* stats);
 
   // Serving (RenderServer): ServePrepare checks the TF slot for `mode`,
-  // uploads TFs and builds the slot's empty-cell flags (device work on this
+  // uploads TFs and builds the slot's cell codes (device work on this
   // renderer's stream is finished when it returns); ServeJob builds the job
   // of one view in `mode` (finest LOD limit) and its kernel variant.
   int ServePrepare(uint32_t tf_slot, int mode);

@@ -14,9 +14,11 @@
 //   cell ranges  uint32 (min | max << 16) per empty-space cell of edge C
 //                (C divides the brick size), over the voxels
 //                [c*C - 1, (c+1)*C] that trilinear samples in the cell read.
-//   cell flags   uint8 per cell and TF slot: 1 when the TF is transparent
-//                over the cell's range (rebuilt when the TF, mode or the
-//                cell ranges change).
+//   cell codes   uint8 per cell and TF slot: bit 0 set when the TF is
+//                transparent over the cell's range, above it the level of the
+//                largest aligned block of cells around it that is all so or
+//                all not (rebuilt when the TF, mode or the cell ranges
+//                change).
 //   TF           n_tf float4 (RGBA) + int32 prefix count of alpha > 0.
 //   framebuffer  W*H uint32 RGBA8 (r in the low byte), row 0 at the top.
 #pragma once
@@ -153,7 +155,7 @@ struct RaycastParams {
   const uint64_t* page_table;   // per brick: device address of its slot, 0 when not resident
   const float* brick_range;     // 2 floats per brick
   const uint32_t* cell_range;   // per cell: min | max << 16 (raw values)
-  const uint8_t* cell_empty;    // per cell: 1 when this job's TF is transparent over it
+  const uint8_t* cell_code;     // per cell: bit 0 this job's TF is transparent over it, above: block level
   int32_t cell;                 // march unit edge in level voxels (divides brick)
   const float* tf;              // 4 floats per entry
   const int32_t* tf_prefix;     // n_tf + 1

@@ -379,3 +379,42 @@ def test_cell_ranges_beyond_one_work_group_per_cell():
     assert np.array_equal(on, off)
     assert s_on <= s_off
     r.cleanup()
+
+
+@pytest.mark.parametrize("dims,brick,cell", [
+    ((70, 45, 33), 32, 4),     # 8 cells a brick: blocks up to 8 cells, partial bricks
+    ((97, 61, 50), 48, 16),    # 3 cells a brick: no aligned block divides it
+    ((150, 33, 70), 64, 4),    # 16 cells a brick: a whole brick may be one block
+    ((40, 41, 150), 32, 16),   # 2 cells a brick, regions of 16^3 cells cut by the level's end
+    ((270, 20, 20), 256, 8),   # 32 cells a brick: blocks stop at 16 cells
+])
+def test_cell_blocks_skip_exactly(dims, brick, cell):
+    """Cells crossed in blocks (all empty or none): the image is the one
+    without skipping, and the samples evaluated are those outside empty
+    cells."""
+    print(f"case cell blocks {dims} brick {brick} cell {cell}", flush=True)
+    nx, ny, nz = dims
+    rng = np.random.default_rng(nx)
+    vol = np.zeros((nz, ny, nx), np.uint8)
+    for _ in range(6):  # boxes of matter in empty space
+        a = [int(rng.integers(0, n)) for n in (nz, ny, nx)]
+        b = [v + int(rng.integers(3, 24)) for v in a]
+        vol[a[0]:b[0], a[1]:b[1], a[2]:b[2]] = rng.integers(150, 255)
+    tf = np.zeros((256, 4), np.float32)
+    tf[140:] = (0.9, 0.6, 0.3, 0.04)
+    w = workloads.Workload("blocks", dims, 8, 0, 0, brick, 2, 1, tf, 160, 120, 1.4,
+                           [Camera((1.2, 0.5, 1.3), (-1.2, -0.5, -1.3), fov=45.0)])
+    r = gpu_renderer(w)
+    r.setEmptySpaceCell(cell)
+    r.setVolume(vol, brick, w.apron, 1)
+    r.set1DTrans(tf)
+    a, sa = render_gpu(r, w, w.cameras[0])
+    w.skip = False
+    b, sb = render_gpu(r, w, w.cameras[0])
+    assert np.array_equal(a, b)
+    assert 0 < sa.evaluated_samples < sb.evaluated_samples
+    # the oracle counts the samples outside empty cells of the same edge;
+    # the slack is the rounding of sample positions at cell faces
+    _, ns, _, _ = oracle_ref(vol, w, w.cameras[0], brick_size=cell, apron=1)
+    assert abs(int(sa.evaluated_samples) - int(ns.sum())) <= 2e-3 * ns.sum() + 64
+    r.cleanup()
