@@ -329,15 +329,16 @@ __device__ inline void tf2d_lookup(const RaycastParams& P, float v, float gm, fl
   const float fx = x - (float)i, fy = y - (float)j;
   const int i1 = min(i + 1, W - 1), j1 = min(j + 1, H - 1);
   const float4* t = (const float4*)P.tf2d;
-  const float4 a = gload_f4(t + (j * W + i)), b = gload_f4(t + (j * W + i1));
-  const float4 e = gload_f4(t + (j1 * W + i)), f = gload_f4(t + (j1 * W + i1));
+  const uint32_t r0 = __umul24((uint32_t)j, (uint32_t)W), r1 = __umul24((uint32_t)j1, (uint32_t)W);
+  const float4 a = gload_f4(t + (r0 + (uint32_t)i)), b = gload_f4(t + (r0 + (uint32_t)i1));
+  const float4 e = gload_f4(t + (r1 + (uint32_t)i)), f = gload_f4(t + (r1 + (uint32_t)i1));
   const float ax[4] = {a.x, a.y, a.z, a.w}, bx[4] = {b.x, b.y, b.z, b.w};
   const float ex[4] = {e.x, e.y, e.z, e.w}, fx4[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float r0 = fmaf(bx[k] - ax[k], fx, ax[k]);
-    const float r1 = fmaf(fx4[k] - ex[k], fx, ex[k]);
-    c[k] = fmaf(r1 - r0, fy, r0);
+    const float c0 = fmaf(bx[k] - ax[k], fx, ax[k]);
+    const float c1 = fmaf(fx4[k] - ex[k], fx, ex[k]);
+    c[k] = fmaf(c1 - c0, fy, c0);
   }
 }
 
@@ -1051,7 +1052,7 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
 }
 
 // The march unit of sample k on a TF group's ray (render_tile_group and
-// render_tile_group_runs), as render_tile's walk finds it: its end kend,
+// render_tile_group_quad), as render_tile's walk finds it: its end kend,
 // the live members whose TF keeps it (need), its brick slot `base` and the
 // slot-local texel origin g0.  Rounds each live member's blend when the
 // brick changes (a member's own march stops rounding once it has
@@ -1632,30 +1633,67 @@ __global__ __launch_bounds__(256) void upscale_nearest_kernel(const uint32_t* __
   }
 }
 
-// Gradient march of a TF group in runs (kModeGradGroup at a gather batch of
-// kRun): the group march above, with the samples gathered by lanes other
-// than the ray's.  Rays about 2 voxels apart (1080p over a 2048-voxel
-// volume) touch a cache line per lane in every voxel gather; here each
-// lane walks its own ray to its next unit with samples to gather, as
-// render_tile_group does, and then the wave gathers in 4 passes: in pass
-// p, lane l takes sample (l & 3) of the run of ray 16p + (l >> 2) -- kRun
-// consecutive samples, 2/3 of a voxel apart, of one ray per 4 lanes, which
-// share their lines -- looks up every member's TF, shades, and leaves
-// (colour, opacity-corrected alpha) per member in the wave's LDS slab
-// (kRun passes of 64 / kRun rays in general);
-// the ray's own lane then composites its run member by member in sample
-// order.  Sample positions, values, lookups and the compositing arithmetic
-// are those of render_tile_group, and a member's samples and termination
-// are its own, so images and counts are the same bit for bit.  Every lane
-// takes part in the passes, rays finished or not; the loop ends when no
-// lane has a run left (a wave-wide ballot).
-constexpr int kRun = 4;
+// The value that lane S of this lane's quad (four consecutive lanes) holds.
+template <int S>
+__device__ inline float quad_lane(float x) {
+  constexpr int kPerm = S * 0x55;  // quad_perm [S, S, S, S]
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kPerm, 0xf, 0xf, true));
+}
+
+// Composites the quad's four consecutive samples (c, opacity-corrected
+// alpha ac; one per lane, sample S on lane S) into the ray's (C, A) in
+// order, on every lane of the quad alike.  live: the ray has not terminated;
+// cnt counts the samples composited while it had not.  A sample with ac = 0
+// leaves (C, A) as they are, as skipping it does.
+template <int S>
+__device__ inline void quad_step(const float (&c)[3], float ac, float term, float (&C)[3], float& A, bool& live,
+                                 uint32_t& cnt) {
+  cnt += live ? 1u : 0u;
+  const float w = live ? (1.f - A) * quad_lane<S>(ac) : 0.f;
+  C[0] = fmaf(w, quad_lane<S>(c[0]), C[0]);
+  C[1] = fmaf(w, quad_lane<S>(c[1]), C[1]);
+  C[2] = fmaf(w, quad_lane<S>(c[2]), C[2]);
+  A += w;
+  live = live && A < term;
+}
+__device__ inline void quad_composite(const float (&c)[3], float ac, float term, float (&C)[3], float& A, bool& live,
+                                      uint32_t& cnt) {
+  quad_step<0>(c, ac, term, C, A, live, cnt);
+  quad_step<1>(c, ac, term, C, A, live, cnt);
+  quad_step<2>(c, ac, term, C, A, live, cnt);
+  quad_step<3>(c, ac, term, C, A, live, cnt);
+}
+
+// The pixel order of a quad wave: it renders a quarter of a ray tile (`sub`,
+// 16 consecutive lanes of the tile's Z order: a 4 x 4 pixel block), ray
+// lane / 4 on the four lanes of each quad.  All four lanes hold the same ray
+// and walk it alike; they gather four consecutive samples of it, one each,
+// 1 / rate of a voxel apart and so mostly on the same cache lines, look them
+// up and shade them, and composite all four in order with values passed by
+// DPP.
+constexpr int kQuad = 4;       // lanes, and samples per gather, of a ray
+constexpr int kQuadSubs = 4;   // quad waves per ray tile
+
+// Gradient march of a TF group, four lanes per ray (kModeGradGroup at a
+// gather batch of kQuad): the group march above with each ray's samples
+// gathered by its quad.  Sample positions, values, lookups and the
+// compositing arithmetic are those of render_tile_group, and a member's
+// samples and termination are its own, so images and counts are the same
+// bit for bit.  n_eval, n_walk and n_nom are counted on the quad's first
+// lane.  Against 64 rays a wave whose runs of 4 samples were gathered in
+// four passes (ray state by cross-lane shuffles, results through LDS): a
+// quarter of the serial chain per wave and no shuffles or LDS.  Lit 720p
+// frame of a u8 scan alone 727 -> 333 us, in a row 306 -> 237; 16 lit 2D-TF
+// views of 1 GiB 24.6 -> 23.2 ms, bound by the 16 voxel and 4 texel gathers.
 template <typename T, bool LINEAR>
-__device__ inline void render_tile_group_runs(const JobTable* __restrict__ tab, const RaycastParams& P,
-                                              int tile, int lane, uint32_t (&n_eval)[kGroupMax],
-                                              uint32_t& n_walk, uint32_t& n_nom, float4* __restrict__ slab) {
-  Ray r = {};
-  const bool mine = setup_ray(P, tile, lane, r, n_nom);
+__device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, const RaycastParams& P,
+                                              int tile, int sub, int lane, uint32_t (&n_eval)[kGroupMax],
+                                              uint32_t& n_walk, uint32_t& n_nom) {
+  const int q = lane & (kQuad - 1);
+  Ray r;
+  uint32_t nom = 0;
+  if (!setup_ray(P, tile, sub * (64 / kQuadSubs) + lane / kQuad, r, nom)) return;
+  if (q == 0) n_nom += nom;
   const int F = P.group_n > 1 ? P.group_n : 1;
   const RaycastParams* Q[kGroupMax];
   Q[0] = &P;
@@ -1664,137 +1702,95 @@ __device__ inline void render_tile_group_runs(const JobTable* __restrict__ tab, 
   float C[kGroupMax][3], A[kGroupMax];
 #pragma unroll
   for (int f = 0; f < kGroupMax; ++f) C[f][0] = C[f][1] = C[f][2] = A[f] = 0.f;
-  const float step = P.step;
   const float t0 = r.t0, L = r.t1 - r.t0;
-  const int n = (mine && r.hit && L > 0.f) ? (int)ceilf(L / step) : 0;
-  const float lastlen = n > 0 ? fmaxf(L - (float)(n - 1) * step, 0.f) : 0.f;
-  const LodInfo& lv = P.level;
-  const Walk walk = make_walk(P, lv, r.o, r.d);
-  const float(&od)[3] = walk.od;
-  const SlotGeo G = slot_geo(P.slot_edge);
-  uint32_t live = n > 0 ? (1u << F) - 1 : 0u;  // members still compositing
-  uint32_t need = 0;                           // live members whose TF keeps the current unit
-  int k = 0, kend = 0, blend_gid = -1;
-  float g0[3] = {0.f, 0.f, 0.f};
-  const T* __restrict__ base = nullptr;
-  while (true) {
-    // this lane's ray: on to the next unit with samples to gather
-    bool ready = false;
-    while (live && k < n) {
-      if (k < kend) {
-        ready = true;
-        break;
-      }
-      if (!group_unit<T, LINEAR>(P, Q, F, r, walk, k, n, t0, step, lastlen, live,
-                                 kend, need, base, g0, blend_gid, C, A))
-        k = kend;
-    }
-    if (__ballot(ready) == 0) break;  // wave-uniform: every lane reaches it
-    const int cnt = ready ? min(kRun, kend - k) : 0;
-    const uint32_t run_need = ready ? need : 0u;
-    const int ib0 = (int)(uint32_t)(uint64_t)base, ib1 = (int)(uint32_t)((uint64_t)base >> 32);
-    constexpr int kRays = 64 / kRun;  // rays whose runs a pass gathers
-    for (int p = 0; p < kRun; ++p) {
-      // this lane gathers sample q of the run of ray `src`
-      const int src = kRays * p + lane / kRun, q = lane % kRun;
-      const int s_cnt = __shfl(cnt, src, 64);
-      const uint32_t s_need = (uint32_t)__shfl((int)run_need, src, 64);
-      const int s_k = __shfl(k, src, 64), s_n = __shfl(n, src, 64);
-      const float s_t0 = __shfl(t0, src, 64), s_last = __shfl(lastlen, src, 64);
-      float s_od[3], s_g0[3], s_d[3];
+  if (r.hit && L > 0.f) {
+    const float step = P.step;
+    const int n = (int)ceilf(L / step);
+    const float lastlen = fmaxf(L - (float)(n - 1) * step, 0.f);
+    const LodInfo& lv = P.level;
+    const Walk walk = make_walk(P, lv, r.o, r.d);
+    const float(&od)[3] = walk.od;
+    const SlotGeo G = slot_geo(P.slot_edge);
+    float Lh[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // light direction, half vector
+    {
+      float h[3], hl = 0.f;
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        s_od[i] = __shfl(od[i], src, 64);
-        s_g0[i] = __shfl(g0[i], src, 64);
-        s_d[i] = __shfl(r.d[i], src, 64);
+        Lh[i] = P.light[i];
+        h[i] = P.light[i] - r.d[i];
+        hl += h[i] * h[i];
       }
-      const uint64_t sb = (uint64_t)(uint32_t)__shfl(ib0, src, 64) | (uint64_t)(uint32_t)__shfl(ib1, src, 64) << 32;
-      if (q < s_cnt) {
-        const T* __restrict__ sbase = (const T*)sb;
-        const int kk = s_k + q;
-        const float len = (kk == s_n - 1) ? s_last : step;
-        const float t = fmaf((float)kk, step, s_t0) + 0.5f * len;
-        const float gx = fmaf(t, s_od[0], s_g0[0]), gy = fmaf(t, s_od[1], s_g0[1]), gz = fmaf(t, s_od[2], s_g0[2]);
-        float v, dd[3];
-        if (LINEAR) {
-          fetch_value_grad<T>(sbase, G, gx, gy, gz, v, dd);
-        } else {
-          v = fetch<T, false>(sbase, G, gx, gy, gz);
-          const float lx = gx - 0.5f, ly = gy - 0.5f, lz = gz - 0.5f;
-          dd[0] = fetch<T, true>(sbase, G, lx + 1.f, ly, lz) - fetch<T, true>(sbase, G, lx - 1.f, ly, lz);
-          dd[1] = fetch<T, true>(sbase, G, lx, ly + 1.f, lz) - fetch<T, true>(sbase, G, lx, ly - 1.f, lz);
-          dd[2] = fetch<T, true>(sbase, G, lx, ly, lz + 1.f) - fetch<T, true>(sbase, G, lx, ly, lz - 1.f);
-        }
-        float g[3] = {dd[0] * P.grad_scale[0], dd[1] * P.grad_scale[1], dd[2] * P.grad_scale[2]};
-        const float gm = sqrtf(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
-        // the source ray's light direction and half vector, as its own march sets them up
-        float Lh[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        {
-          float h[3], hl = 0.f;
+      hl = sqrtf(hl);
+      if (hl > 1e-12f)
 #pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            Lh[i] = P.light[i];
-            h[i] = P.light[i] - s_d[i];
-            hl += h[i] * h[i];
-          }
-          hl = sqrtf(hl);
-          if (hl > 1e-12f)
-#pragma unroll
-            for (int i = 0; i < 3; ++i) Lh[3 + i] = h[i] / hl;
-        }
-#pragma unroll
-        for (int f = 0; f < kGroupMax; ++f) {
-          if (!(s_need >> f & 1u)) continue;
-          float cs[4];
-          if (P.mode == 1) tf2d_lookup(*Q[f], v, gm, cs);
-          else tf1d_lookup<false>(*Q[f], (const float4*)Q[f]->tf, v, cs);
-          float ac = 0.f;  // compositing with 0 leaves (C, A) as skipping the sample does
-          if (cs[3] > 0.f) {
-            if (P.lighting) shade(P, g, Lh, cs);
-            ac = step_opacity(cs[3], len);
-          }
-          slab[f * 64 + lane] = make_float4(cs[0], cs[1], cs[2], ac);
-        }
-      }
-      wave_lds_sync();
-      if (lane / kRays == p && cnt > 0) {
-        // this lane's ray was gathered in this pass by lanes kRun (lane - kRays p) + q
-        const int w0 = kRun * (lane - kRays * p);
-        int most = 0;  // samples of the run some member evaluates
-#pragma unroll
-        for (int f = 0; f < kGroupMax; ++f) {
-          if (!(run_need >> f & 1u)) continue;
-          int e = 0;
-          for (int j = 0; j < cnt && (live >> f & 1u); ++j) {
-            const float4 x = slab[f * 64 + w0 + j];
-            ++e;
-            const float w = (1.f - A[f]) * x.w;
-            C[f][0] = fmaf(w, x.x, C[f][0]);
-            C[f][1] = fmaf(w, x.y, C[f][1]);
-            C[f][2] = fmaf(w, x.z, C[f][2]);
-            A[f] += w;
-            if (!(A[f] < P.term_alpha)) {
-              live &= ~(1u << f);
-              need &= ~(1u << f);
-            }
-          }
-          n_eval[f] += (uint32_t)e;
-          most = max(most, e);
-        }
-        n_walk += (uint32_t)most;
-      }
-      wave_lds_sync();  // the slab is the next pass's
+        for (int i = 0; i < 3; ++i) Lh[3 + i] = h[i] / hl;
     }
-    if (ready) k = live ? (need ? k + cnt : kend) : n;
-  }
-  if (n > 0 && P.blend_bits < 32)
+    uint32_t live = (1u << F) - 1;  // members still compositing
+    uint32_t need = 0;              // live members whose TF keeps the current unit
+    int k = 0, kend = 0, blend_gid = -1;
+    float g0[3] = {0.f, 0.f, 0.f};
+    const T* __restrict__ base = nullptr;
+    while (k < n) {  // alike on a quad's lanes
+      if (k >= kend && !group_unit<T, LINEAR>(P, Q, F, r, walk, k, n, t0, step, lastlen, live, kend, need, base, g0,
+                                              blend_gid, C, A)) {
+        k = kend;
+        continue;
+      }
+      const int cnt = min(kQuad, kend - k);
+      // this lane's sample; a lane past the unit's end gathers its last one
+      // again and composites nothing
+      const int kk = min(k + q, kend - 1);
+      const float len = (kk == n - 1) ? lastlen : step;
+      const float t = fmaf((float)kk, step, t0) + 0.5f * len;
+      const float gx = fmaf(t, od[0], g0[0]), gy = fmaf(t, od[1], g0[1]), gz = fmaf(t, od[2], g0[2]);
+      float v, dd[3];
+      if (LINEAR) {
+        fetch_value_grad<T>(base, G, gx, gy, gz, v, dd);
+      } else {
+        v = fetch<T, false>(base, G, gx, gy, gz);
+        const float lx = gx - 0.5f, ly = gy - 0.5f, lz = gz - 0.5f;
+        dd[0] = fetch<T, true>(base, G, lx + 1.f, ly, lz) - fetch<T, true>(base, G, lx - 1.f, ly, lz);
+        dd[1] = fetch<T, true>(base, G, lx, ly + 1.f, lz) - fetch<T, true>(base, G, lx, ly - 1.f, lz);
+        dd[2] = fetch<T, true>(base, G, lx, ly, lz + 1.f) - fetch<T, true>(base, G, lx, ly, lz - 1.f);
+      }
+      const float g[3] = {dd[0] * P.grad_scale[0], dd[1] * P.grad_scale[1], dd[2] * P.grad_scale[2]};
+      const float gm = sqrtf(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
+      uint32_t most = 0;  // samples of the four that some member evaluates
 #pragma unroll
-    for (int f = 0; f < kGroupMax; ++f) blend_round(P.blend_bits, C[f][0], C[f][1], C[f][2], A[f]);
-  if (!mine) return;
+      for (int f = 0; f < kGroupMax; ++f) {
+        if (!(need >> f & 1u)) continue;
+        float cs[4];
+        if (P.mode == 1) tf2d_lookup(*Q[f], v, gm, cs);
+        else tf1d_lookup<false>(*Q[f], (const float4*)Q[f]->tf, v, cs);
+        float ac = 0.f;
+        if (q < cnt && cs[3] > 0.f) {
+          if (P.lighting) shade(P, g, Lh, cs);
+          ac = step_opacity(cs[3], len);
+        }
+        const float c[3] = {cs[0], cs[1], cs[2]};
+        bool on = true;
+        uint32_t e = 0;
+        quad_composite(c, ac, P.term_alpha, C[f], A[f], on, e);
+        e = min(e, (uint32_t)cnt);  // past the unit's end nothing terminates
+        if (q == 0) n_eval[f] += e;
+        most = max(most, e);
+        if (!on) {
+          live &= ~(1u << f);
+          need &= ~(1u << f);
+        }
+      }
+      if (q == 0) n_walk += most;
+      k = need ? k + cnt : (live ? kend : n);
+    }
+    if (P.blend_bits < 32)
+#pragma unroll
+      for (int f = 0; f < kGroupMax; ++f) blend_round(P.blend_bits, C[f][0], C[f][1], C[f][2], A[f]);
+  }
   const int64_t pix = (int64_t)r.py * P.width + r.px;
 #pragma unroll
   for (int f = 0; f < kGroupMax; ++f)
-    if (f < F) gstore(Q[f]->framebuffer + pix, over_background(P, r.py, C[f][0], C[f][1], C[f][2], A[f]));
+    if (f < F && q == (f & (kQuad - 1)))
+      gstore(Q[f]->framebuffer + pix, over_background(P, r.py, C[f][0], C[f][1], C[f][2], A[f]));
 }
 
 // Persistent raycast over a job table: every wave loops over ray tiles
@@ -1819,6 +1815,9 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
   const int n_jobs = H.n_jobs;
   const int total = H.total_tiles;
   const int G = H.tile_group;
+  // quad waves take a quarter of a ray tile per ticket
+  constexpr int kSubShift = (MODE == kModeGradGroup && BATCH == kQuad) ? 2 : 0;
+  static_assert(1 << 2 == kQuadSubs, "a quad ticket is tile * kQuadSubs + quarter");
   // xcd_split regions apply to one-job launches only
   const int split = n_jobs == 1 ? H.xcd_split : 0;
   const int tiles_x0 = tab->jobs[0].rect_w, tiles_y0 = tab->jobs[0].rect_h;
@@ -1881,7 +1880,8 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
       // that the compiler could split off the loop around the wave-wide
       // broadcast of the ticket.
       const unsigned long long ticket = wave_atomic_add(&queues[x * kQueueStride], lane == 0 ? 1ull : 0ull);
-      const int pos = __builtin_amdgcn_readfirstlane((int)__shfl((long long)ticket, 0, 64));
+      const int at = __builtin_amdgcn_readfirstlane((int)__shfl((long long)ticket, 0, 64));
+      const int pos = at >> kSubShift;
       if (pos >= slots) break;
       int tile;
       if (split == 0) tile = ((pos / G) * 8 + x) * G + (pos % G);
@@ -1908,11 +1908,8 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
         // this wave's staging buffer follows the LDS TF
         T* sbuf = (T*)(s_tf + (TF_LDS ? H.n_tf_lds + 1 : 0)) + (threadIdx.x >> 6) * kStageElems;
         render_tile_staged<T, TF_LDS>(P, tf4, slot, lane, n_eval, n_nom, sbuf);
-      } else if constexpr (MODE == kModeGradGroup && BATCH == kRun) {
-        // this wave's slab follows the work-group's counters in LDS
-        float4* slab = s_tf + (threadIdx.x >> 6) * 64 * kGroupMax;
-        render_tile_group_runs<T, LINEAR>(tab, P, slot, lane, n_evalg, n_walk, n_nom,
-                                          slab);
+      } else if constexpr (MODE == kModeGradGroup && BATCH == kQuad) {
+        render_tile_group_quad<T, LINEAR>(tab, P, slot, at & (kQuadSubs - 1), lane, n_evalg, n_walk, n_nom);
       } else if constexpr (MODE == kModeGradGroup) {
         render_tile_group<T, LINEAR, BATCH>(tab, P, slot, lane, n_evalg, n_walk, n_nom);
       } else {
@@ -1932,7 +1929,7 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
     const int qslots = region(qx, ux0, uw, uy0);
     const unsigned long long head = __hip_atomic_load((global_u64*)&queues[qx * kQueueStride], __ATOMIC_RELAXED,
                                                       __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t open = (uint32_t)(__ballot(head < (unsigned long long)qslots) & 0xffull);
+    const uint32_t open = (uint32_t)(__ballot(head < (unsigned long long)qslots << kSubShift) & 0xffull);
     if (open == 0) break;
     const uint32_t ahead = ((open | open << 8) >> x) & 0xffu;  // bit k: queue (x + k) & 7 has tiles
     x = (x + __builtin_ctz(ahead)) & 7;
@@ -1957,7 +1954,6 @@ hipError_t launch_one(const LaunchInfo& li, const JobTable* tab, hipStream_t str
   // in flight thrash the caches (the autotuner picks).
   const int kT = TF_LDS ? kThreads : 64 * (li.wg_waves == 4 ? 4 : 8);
   if (MODE == kMode1DStaged) lds += (size_t)(kT / 64) * kStageElems * sizeof(T);  // per-wave cell buffers
-  if (MODE == kModeGradGroup && BATCH == kRun) lds += (size_t)(kT / 64) * 64 * kGroupMax * sizeof(float4);
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kT, lds);
   if (e != hipSuccess) return e;
   if (per_cu < 1) per_cu = 1;
@@ -1986,13 +1982,12 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
     return li.n_tf_lds > 0 ? launch_one<T, LINEAR, 4, true, kModeMIP>(li, tab, stream)
                            : launch_one<T, LINEAR, 4, false, kModeMIP>(li, tab, stream);
   // the gradient marches: li.batch 1 or 2 samples per gather batch, each
-  // lane its own ray; otherwise runs of kRun samples per ray gathered
-  // across lanes (the TF-group march, which takes lone views as groups of
-  // one)
+  // lane its own ray; otherwise four lanes per ray, a sample each (the
+  // TF-group march, which takes lone views as groups of one)
   if (li.mode == 1 || li.lighting) {
     if (li.batch == 1) return launch_grad<T, LINEAR, 1>(li, tab, stream);
     if (li.batch == 2) return launch_grad<T, LINEAR, 2>(li, tab, stream);
-    return launch_one<T, LINEAR, kRun, false, kModeGradGroup>(li, tab, stream);
+    return launch_one<T, LINEAR, kQuad, false, kModeGradGroup>(li, tab, stream);
   }
   const bool lds = li.n_tf_lds > 0;
   if (li.stage && LINEAR && !li.lighting)
