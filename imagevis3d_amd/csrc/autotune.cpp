@@ -87,15 +87,17 @@ int HipRenderer::Autotune(const tvk_view* views, uint32_t n, uint32_t flags, tvk
   // then the launch shape again for the chosen bricks: tuning the bricks
   // under the starting launch shape can settle on bricks that are only best
   // for that shape.
-  // samples per gather batch: 2, 4 or 8 for the 1D march; for the gradient
-  // marches (2D TF, or 1D TF with lighting) 1 or 2 per lane, or 4 = runs of
-  // 4 samples per ray gathered across lanes; the other modes' batch is
-  // fixed
+  // samples per gather batch: 2 or 4 for the 1D march, 8 too with nearest
+  // sampling (trilinear runs 8 as 4); for the gradient marches (2D TF, or 1D
+  // TF with lighting) 1 or 2 per lane, or 4 = four lanes per ray; the other
+  // modes' batch is fixed
   const int mode = job_mode();
   const bool grad = mode == 1 || (mode == 0 && lighting_);
   const std::vector<uint32_t> batches =
       grad ? std::vector<uint32_t>{1u, 2u, 4u}
-           : (mode == 0 && !regions_active() ? std::vector<uint32_t>{2u, 4u, 8u} : std::vector<uint32_t>{});
+           : (mode != 0 || regions_active() ? std::vector<uint32_t>{}
+                 : interp_ == TVK_LINEAR    ? std::vector<uint32_t>{2u, 4u}
+                                            : std::vector<uint32_t>{2u, 4u, 8u});
   auto tune_launch = [&]() -> int {
     if (int e = try_values(batches, &Setting::batch, false)) return e;
     if (int e = try_values({4u, 8u, 16u}, &Setting::tile_width, false)) return e;
