@@ -320,14 +320,27 @@ __device__ inline void tf1d_lookup(const RaycastParams& P, const float4* __restr
   c[3] = fmaf(e1.w - e0.w, f, e0.w);
 }
 
-// 2D TF (value x gradient magnitude), bilinear, value fastest.
-__device__ inline void tf2d_lookup(const RaycastParams& P, float v, float gm, float c[4]) {
+// 2D TF (value x gradient magnitude), bilinear, value fastest.  A texel cell
+// without any alpha > 0 (its bit in the TF's mask, from LDS when the launch
+// staged it) is transparent whatever its colours, and its four 16-byte
+// texels are not read (a 16-byte gather of 64 lanes costs the vector-memory
+// path about 64 cycles, an x-pair's 27).  16 lit 2D-TF views of 1 GiB 23.2 ->
+// 21.8 ms, 24 served requests 11.2 -> 10.4; a small 1D TF in LDS instead: a
+// lit 720p frame 237 -> 225 us.
+__device__ inline void tf2d_lookup(const RaycastParams& P, const float4* __restrict__ lds, float v, float gm,
+                                   float c[4]) {
   const int W = P.tf2d_w, H = P.tf2d_h;
   const float x = __builtin_amdgcn_fmed3f(v * P.tf_scale, 0.f, (float)(W - 1));
   const float y = __builtin_amdgcn_fmed3f(gm * P.tf2d_row_scale, 0.f, (float)(H - 1));
   const int i = (int)x, j = (int)y;
   const float fx = x - (float)i, fy = y - (float)j;
   const int i1 = min(i + 1, W - 1), j1 = min(j + 1, H - 1);
+  const uint32_t bit = __umul24((uint32_t)j, (uint32_t)W) + (uint32_t)i;
+  const uint32_t word = P.lds_at >= 0 ? ((const uint32_t*)(lds + P.lds_at))[bit >> 5] : gload(P.tf2d_mask + (bit >> 5));
+  if (!(word >> (bit & 31u) & 1u)) {
+    c[0] = c[1] = c[2] = c[3] = 0.f;
+    return;
+  }
   const float4* t = (const float4*)P.tf2d;
   const uint32_t r0 = __umul24((uint32_t)j, (uint32_t)W), r1 = __umul24((uint32_t)j1, (uint32_t)W);
   const float4 a = gload_f4(t + (r0 + (uint32_t)i)), b = gload_f4(t + (r0 + (uint32_t)i1));
@@ -340,6 +353,15 @@ __device__ inline void tf2d_lookup(const RaycastParams& P, float v, float gm, fl
     const float c1 = fmaf(fx4[k] - ex[k], fx, ex[k]);
     c[k] = fmaf(c1 - c0, fy, c0);
   }
+}
+
+// A gradient launch's TF lookup: 2D by value and gradient magnitude, or 1D
+// from LDS when the launch staged the job's table, else from memory.
+__device__ inline void tf_lookup(const RaycastParams& P, const float4* __restrict__ lds, float v, float gm,
+                                 float c[4]) {
+  if (P.mode == 1) tf2d_lookup(P, lds, v, gm, c);
+  else if (P.lds_at >= 0) tf1d_lookup<true>(P, lds + P.lds_at, v, c);
+  else tf1d_lookup<false>(P, (const float4*)P.tf, v, c);
 }
 
 // Two-sided Blinn-Phong: c*(ka + kd|N.L|) + ks|N.H|^shininess with
@@ -712,7 +734,8 @@ __device__ inline int unit_end(const Walk& w, const float (&o)[3], const float (
 }
 
 template <typename T, bool LINEAR, int BATCH, int MODE, bool TF_LDS>
-__device__ inline void render_tile(const RaycastParams& P, const float4* __restrict__ tf4, int tile,
+__device__ inline void render_tile(const RaycastParams& P, const float4* __restrict__ tf4,
+                                   const float4* __restrict__ lds, int tile,
                                    int lane, uint32_t& n_eval, uint32_t& n_nom) {
   Ray r;
   if (!setup_ray(P, tile, lane, r, n_nom)) return;
@@ -873,11 +896,11 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
           if (k + j < kend && live) {
             ++n_eval;
             float cs[4];
-            if (P.mode == 1) {
-              const float gm = sqrtf(g[j][0] * g[j][0] + g[j][1] * g[j][1] + g[j][2] * g[j][2]);
-              tf2d_lookup(P, v[j], gm, cs);
+            if constexpr (TF_LDS) {  // a launch of one 1D TF
+              tf1d_lookup<true>(P, tf4, v[j], cs);
             } else {
-              tf1d_lookup<TF_LDS>(P, tf4, v[j], cs);
+              const float gm = sqrtf(g[j][0] * g[j][0] + g[j][1] * g[j][1] + g[j][2] * g[j][2]);
+              tf_lookup(P, lds, v[j], gm, cs);
             }
             if (cs[3] > 0.f) {
               if (P.lighting) shade(P, g[j], Lh, cs);
@@ -1113,7 +1136,8 @@ __device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* c
 // path with one TF.  n_eval[f] counts member f's samples, n_walk the
 // samples of the walk that some member evaluates (the union of theirs).
 template <typename T, bool LINEAR, int BATCH>
-__device__ inline void render_tile_group(const JobTable* __restrict__ tab, const RaycastParams& P, int tile,
+__device__ inline void render_tile_group(const JobTable* __restrict__ tab, const RaycastParams& P,
+                                         const float4* __restrict__ lds, int tile,
                                          int lane, uint32_t (&n_eval)[kGroupMax], uint32_t& n_walk,
                                          uint32_t& n_nom) {
   Ray r;
@@ -1190,8 +1214,7 @@ __device__ inline void render_tile_group(const JobTable* __restrict__ tab, const
           if (!(need >> f & 1u)) continue;
           ++n_eval[f];
           float cs[4];
-          if (P.mode == 1) tf2d_lookup(*Q[f], v[j], gm, cs);
-          else tf1d_lookup<false>(*Q[f], (const float4*)Q[f]->tf, v[j], cs);
+          tf_lookup(*Q[f], lds, v[j], gm, cs);
           if (cs[3] > 0.f) {
             if (P.lighting) shade(P, g[j], Lh, cs);
             const float ac = step_opacity(cs[3], len[j]);
@@ -1687,6 +1710,7 @@ constexpr int kQuadSubs = 4;   // quad waves per ray tile
 // views of 1 GiB 24.6 -> 23.2 ms, bound by the 16 voxel and 4 texel gathers.
 template <typename T, bool LINEAR>
 __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, const RaycastParams& P,
+                                              const float4* __restrict__ lds,
                                               int tile, int sub, int lane, uint32_t (&n_eval)[kGroupMax],
                                               uint32_t& n_walk, uint32_t& n_nom) {
   const int q = lane & (kQuad - 1);
@@ -1760,8 +1784,7 @@ __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, 
       for (int f = 0; f < kGroupMax; ++f) {
         if (!(need >> f & 1u)) continue;
         float cs[4];
-        if (P.mode == 1) tf2d_lookup(*Q[f], v, gm, cs);
-        else tf1d_lookup<false>(*Q[f], (const float4*)Q[f]->tf, v, cs);
+        tf_lookup(*Q[f], lds, v, gm, cs);
         float ac = 0.f;
         if (q < cnt && cs[3] > 0.f) {
           if (P.lighting) shade(P, g, Lh, cs);
@@ -1799,7 +1822,10 @@ __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, 
 template <typename T, bool LINEAR, int BATCH, bool TF_LDS, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __restrict__ tab) {
   const int kT = (int)blockDim.x;  // 256 or 512 threads (see launch_one)
-  extern __shared__ float4 s_tf[];  // n_tf_lds + 1 entries when TF_LDS
+  // TF_LDS: the launch's 1D TF, n_tf_lds + 1 entries; gradient launches
+  // without it: the tables the host chose
+  extern __shared__ float4 s_tf[];
+  constexpr bool kGradTables = !TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup);
   __shared__ unsigned long long s_count[kJobCounters * kMaxJobs];  // per job: evaluated, nominal, gathered
   const JobTableHeader& H = tab->h;
   const float4* tf_shared = (const float4*)H.tf_lds;
@@ -1807,6 +1833,11 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
     for (int i = (int)threadIdx.x; i <= H.n_tf_lds; i += kT) s_tf[i] = tf_shared[i];
     tf_shared = s_tf;
   }
+  if (kGradTables)
+    for (int m = 0; m < H.n_tables; ++m) {
+      const LdsTable tb = H.tables[m];
+      for (int i = (int)threadIdx.x; i < tb.quads; i += kT) s_tf[tb.at + i] = gload_f4((const float4*)tb.src + i);
+    }
   for (int i = (int)threadIdx.x; i < kJobCounters * kMaxJobs; i += kT) s_count[i] = 0;
   __syncthreads();
   const int lane = (int)(threadIdx.x & 63);
@@ -1909,11 +1940,11 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
         T* sbuf = (T*)(s_tf + (TF_LDS ? H.n_tf_lds + 1 : 0)) + (threadIdx.x >> 6) * kStageElems;
         render_tile_staged<T, TF_LDS>(P, tf4, slot, lane, n_eval, n_nom, sbuf);
       } else if constexpr (MODE == kModeGradGroup && BATCH == kQuad) {
-        render_tile_group_quad<T, LINEAR>(tab, P, slot, at & (kQuadSubs - 1), lane, n_evalg, n_walk, n_nom);
+        render_tile_group_quad<T, LINEAR>(tab, P, s_tf, slot, at & (kQuadSubs - 1), lane, n_evalg, n_walk, n_nom);
       } else if constexpr (MODE == kModeGradGroup) {
-        render_tile_group<T, LINEAR, BATCH>(tab, P, slot, lane, n_evalg, n_walk, n_nom);
+        render_tile_group<T, LINEAR, BATCH>(tab, P, s_tf, slot, lane, n_evalg, n_walk, n_nom);
       } else {
-        render_tile<T, LINEAR, BATCH, MODE, TF_LDS>(P, tf4, slot, lane, n_eval, n_nom);
+        render_tile<T, LINEAR, BATCH, MODE, TF_LDS>(P, tf4, s_tf, slot, lane, n_eval, n_nom);
       }
     }
     // This queue is drained: one load per lane looks at all heads, and the
@@ -1953,6 +1984,7 @@ hipError_t launch_one(const LaunchInfo& li, const JobTable* tab, hipStream_t str
   // which is faster on cache-friendly volumes and slower where more waves
   // in flight thrash the caches (the autotuner picks).
   const int kT = TF_LDS ? kThreads : 64 * (li.wg_waves == 4 ? 4 : 8);
+  if (!TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup)) lds += (size_t)li.lds_quads * sizeof(float4);
   if (MODE == kMode1DStaged) lds += (size_t)(kT / 64) * kStageElems * sizeof(T);  // per-wave cell buffers
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kT, lds);
   if (e != hipSuccess) return e;

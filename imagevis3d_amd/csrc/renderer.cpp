@@ -988,6 +988,17 @@ int HipRenderer::Set2DTransSlot(uint32_t slot, const float* rgba, uint32_t w, ui
     for (size_t j = 0; j < h && !any; ++j) any = rgba[4 * (j * w + i) + 3] > 0.f;
     t.prefix2d[i + 1] = t.prefix2d[i] + any;
   }
+  // the texel cells that some texel with alpha > 0 bounds
+  t.mask2d.assign((((size_t)w * h + 127) / 128) * 4, 0u);
+  for (uint32_t j = 0; j < h; ++j)
+    for (uint32_t i = 0; i < w; ++i) {
+      if (!(rgba[4 * ((size_t)j * w + i) + 3] > 0.f)) continue;
+      for (uint32_t y = j > 0 ? j - 1 : 0; y <= j; ++y)
+        for (uint32_t x = i > 0 ? i - 1 : 0; x <= i; ++x) {
+          const size_t b = (size_t)y * w + x;
+          t.mask2d[b >> 5] |= 1u << (b & 31);
+        }
+    }
   t.dirty2d = true;
   ++t.version;
   if (slot == 0) invalidate();
@@ -1096,6 +1107,8 @@ int HipRenderer::upload_tf() {
       const size_t W = t.w2d, H = t.h2d;
       if (t.tf2d_dev.bytes < W * H * 16) TVK_HIP(t.tf2d_dev.alloc(W * H * 16));
       if (t.prefix2d_dev.bytes < (W + 1) * 4) TVK_HIP(t.prefix2d_dev.alloc((W + 1) * 4));
+      if (t.mask2d_dev.bytes < t.mask2d.size() * 4) TVK_HIP(t.mask2d_dev.alloc(t.mask2d.size() * 4));
+      TVK_HIP(hipMemcpyAsync(t.mask2d_dev.p, t.mask2d.data(), t.mask2d.size() * 4, hipMemcpyHostToDevice, stream_));
       TVK_HIP(hipMemcpyAsync(t.tf2d_dev.p, t.tf2d.data(), W * H * 16, hipMemcpyHostToDevice, stream_));
       TVK_HIP(hipMemcpyAsync(t.prefix2d_dev.p, t.prefix2d.data(), (W + 1) * 4, hipMemcpyHostToDevice,
                              stream_));
@@ -1566,6 +1579,7 @@ void HipRenderer::build_params(RaycastParams* p, int lod, const CameraState& cam
   if (p->mode == 1) {
     p->lighting = lighting_ ? 1 : 0;
     p->tf2d = tfs.tf2d_dev.as<float>();
+    p->tf2d_mask = tfs.mask2d_dev.as<uint32_t>();
     p->tf2d_w = (int32_t)tfs.w2d;
     p->tf2d_h = (int32_t)tfs.h2d;
     p->tf2d_row_scale = (float)((double)(tfs.h2d - 1) / (double)tfs.max_grad);
@@ -1620,6 +1634,8 @@ static bool same_but_tf(const RaycastParams& a, const RaycastParams& b) {
   memcpy(&y, &b, sizeof y);
   for (RaycastParams* p : {&x, &y}) {
     p->tf2d = nullptr;
+    p->tf2d_mask = nullptr;
+    p->lds_at = 0;
     p->tf2d_w = p->tf2d_h = 0;
     p->tf2d_row_scale = p->tf_scale = 0.f;
     p->n_tf = 0;
@@ -1640,7 +1656,7 @@ static bool same_but_tf(const RaycastParams& a, const RaycastParams& b) {
 // kGroupMax, the first of them leading); *groups = the groups formed.
 static int fill_job_table(JobTable* t, const RaycastParams* jobs, int n, const LaunchInfo& li,
                           int tile_group, int xcd_split, unsigned long long* dev_counters, bool* culled,
-                          int* groups) {
+                          int* groups, int* lds_quads) {
   t->h.n_jobs = n;
   t->h.tile_group = tile_group;
   t->h.xcd_split = xcd_split;
@@ -1652,6 +1668,28 @@ static int fill_job_table(JobTable* t, const RaycastParams* jobs, int n, const L
     t->jobs[k] = jobs[k];
     t->jobs[k].group_n = 0;
     memset(t->jobs[k].group_jobs, 0, sizeof t->jobs[k].group_jobs);
+    t->jobs[k].lds_at = -1;
+  }
+  // Gradient launches look their TFs up through vector memory, which they
+  // are bound by; the jobs' distinct 2D TF masks (8 KiB at 256 x 256) or
+  // small 1D TFs go to LDS as far as they fit.  32 KiB leave room for the
+  // three 4-wave work-groups per CU that the registers allow.
+  t->h.n_tables = 0;
+  *lds_quads = 0;
+  if (li.mode == 1 || li.lighting) {
+    for (int k = 0; k < n; ++k) {
+      RaycastParams& j = t->jobs[k];
+      const void* src = j.mode == 1 ? (const void*)j.tf2d_mask : (const void*)j.tf;
+      const int64_t quads = j.mode == 1 ? ((int64_t)j.tf2d_w * j.tf2d_h + 127) / 128 : (int64_t)j.n_tf + 1;
+      for (int m = 0; m < t->h.n_tables && j.lds_at < 0; ++m)
+        if (t->h.tables[m].src == src) j.lds_at = t->h.tables[m].at;
+      if (j.lds_at >= 0 || t->h.n_tables == kLdsTables || *lds_quads + quads > kLdsTableQuads) continue;
+      j.lds_at = *lds_quads;
+      t->h.tables[t->h.n_tables++] = LdsTable{src, (int32_t)quads, *lds_quads};
+      *lds_quads += (int)quads;
+    }
+    // whole KiB, so that launches of like TFs share a captured graph
+    *lds_quads = (*lds_quads + 63) / 64 * 64;
   }
   if (li.group) {
     for (int k = 0; k < n; ++k) {
@@ -1691,10 +1729,11 @@ int launch_job_table_at(JobTable* table_h, void* dev_table, unsigned long long* 
                         unsigned long long* counters_h, hipEvent_t ev[4], const RaycastParams* jobs, int n,
                         const LaunchInfo& li_in, int tile_group, int xcd_split, hipStream_t stream_) {
   bool culled = false;  // some job has background tiles outside its rect
-  int groups = 0;
-  fill_job_table(table_h, jobs, n, li_in, tile_group, xcd_split, dev_counters, &culled, &groups);
+  int groups = 0, lds_quads = 0;
+  fill_job_table(table_h, jobs, n, li_in, tile_group, xcd_split, dev_counters, &culled, &groups, &lds_quads);
   LaunchInfo li = li_in;
   li.group = groups > 0 ? 1 : 0;
+  li.lds_quads = lds_quads;
   const int words = kCounterBase + kJobCounters * n;
   const size_t table_bytes = offsetof(JobTable, jobs) + (size_t)n * sizeof(RaycastParams);
   TVK_HIP(hipEventRecord(ev[0], stream_));
@@ -1721,11 +1760,12 @@ int launch_job_table(LaunchSlot& sl, const RaycastParams* jobs, int n, const Lau
                                sl.ev, jobs, n, li_in, tile_group, xcd_split, stream_);
   JobTable* t = sl.table_h;
   bool culled = false;
-  int groups = 0;
+  int groups = 0, lds_quads = 0;
   fill_job_table(t, jobs, n, li_in, tile_group, xcd_split, sl.counters.as<unsigned long long>(), &culled,
-                 &groups);
+                 &groups, &lds_quads);
   LaunchInfo li = li_in;
   li.group = groups > 0 ? 1 : 0;
+  li.lds_quads = lds_quads;
   TVK_HIP(hipEventRecord(sl.ev[0], stream_));
   // Graph replay: the graph copies the whole table and all counters, so one
   // capture serves any job count; it is re-captured when the kernel
@@ -1734,7 +1774,7 @@ int launch_job_table(LaunchSlot& sl, const RaycastParams* jobs, int n, const Lau
                        (uint64_t)li.lighting << 6 | (uint64_t)li.batch << 7 | (uint64_t)li.regions << 11 |
                        (uint64_t)li.n_tf_lds << 12 |
                        (uint64_t)(li.wg_waves == 4 ? 1 : 0) << 40 | (uint64_t)li.stage << 41 |
-                       (uint64_t)li.group << 42;
+                       (uint64_t)li.group << 42 | (uint64_t)(li.lds_quads / 64) << 43;
   if (!sl.exec || sl.graph_key != key) {
     if (sl.exec) (void)hipGraphExecDestroy(sl.exec);
     if (sl.graph) (void)hipGraphDestroy(sl.graph);
@@ -2086,7 +2126,9 @@ bool HipRenderer::launch_ready_without_alloc(const tvk_view* views, uint32_t n, 
     }
     if (t.dirty2d) {
       const size_t W = t.w2d, H = t.h2d;
-      if (t.tf2d_dev.bytes < W * H * 16 || t.prefix2d_dev.bytes < (W + 1) * 4) return false;
+      if (t.tf2d_dev.bytes < W * H * 16 || t.prefix2d_dev.bytes < (W + 1) * 4 ||
+          t.mask2d_dev.bytes < t.mask2d.size() * 4)
+        return false;
     }
   }
   if (skip_ && total_cells_ > 0)
@@ -2361,7 +2403,7 @@ int HipRenderer::MemStats(tvk_mem_stats* out) {
                cell_range_.bytes;
   for (auto& l : levels_) a += l.bytes;
   for (const TfSet& t : tfs_) {
-    a += t.tf1d_dev.bytes + t.prefix1d_dev.bytes + t.tf2d_dev.bytes + t.prefix2d_dev.bytes;
+    a += t.tf1d_dev.bytes + t.prefix1d_dev.bytes + t.tf2d_dev.bytes + t.prefix2d_dev.bytes + t.mask2d_dev.bytes;
     for (const DevBuf& f : t.cell_code) a += f.bytes;
   }
   for (const LaunchSlot* sl : {&paint_slots_[0], &paint_slots_[1], &batch_slot_})

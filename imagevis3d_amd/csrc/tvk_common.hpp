@@ -139,6 +139,12 @@ struct RaycastParams {
   const float* tf2d;    // tf2d_w x tf2d_h float4, value fastest
   int32_t tf2d_w, tf2d_h;
   float tf2d_row_scale; // (tf2d_h - 1) / max gradient
+  // One bit per texel cell (i, j) of the 2D TF, at j * tf2d_w + i: some texel
+  // of (i, j) .. (i + 1, j + 1) has alpha > 0.
+  const uint32_t* tf2d_mask;
+  // Where a gradient launch staged this job's table in LDS, in 16-byte units
+  // (its 2D TF's mask, or its 1D TF); < 0: not staged.
+  int32_t lds_at;
   float iso_value;      // raw data units
   float iso_color[3];
   // ClearView (mode 2, cv != 0): the iso_value surface is the context; in a
@@ -200,14 +206,25 @@ constexpr int kQueues = 8;  // one tile queue per XCD
 // per us for the whole chip, all eight queues together).
 constexpr int kQueueStride = 32;               // u64 words from one head to the next
 constexpr int kCounterBase = kQueues * kQueueStride;  // first word of the jobs' counters
+// A table that a gradient launch's work-groups copy to LDS (16-byte units).
+struct LdsTable {
+  const void* src;
+  int32_t quads;
+  int32_t at;
+};
+constexpr int kLdsTables = 8;
+constexpr int kLdsTableQuads = 2048;  // 32 KiB for all of a launch's tables
+
 struct JobTableHeader {
   int32_t n_jobs;
   int32_t total_tiles;
   int32_t tile_group;   // consecutive ray tiles dealt to one XCD in turn
   int32_t xcd_split;    // one-job launches: 0 round-robin runs; rx: rx x (8/rx) regions
   int32_t n_tf_lds;     // > 0: every job reads this 1D TF, staged into LDS
-  int32_t pad_[3];
+  int32_t n_tables;     // tables[0 .. n_tables) go to LDS (gradient launches)
+  int32_t pad_[2];
   const float* tf_lds;
+  LdsTable tables[kLdsTables];
   // per-XCD tile queue heads every kQueueStride words, then from
   // b = kCounterBase per job j: [b + 3j] evaluated samples, [b + 3j + 1]
   // nominal samples, [b + 3j + 2] gathered samples (those
