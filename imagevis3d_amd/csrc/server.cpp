@@ -474,10 +474,15 @@ void RenderServer::loop() {
   std::unique_lock<std::mutex> lk(mu_);
   while (true) {
     bool progress = retire_locked();
-    for (Lane& L : lanes_)
-      if (!L.busy && !pending_.empty() && !stop_) progress |= launch_locked(L);
     bool busy = false;
     for (const Lane& L : lanes_) busy |= L.busy;
+    for (Lane& L : lanes_) {
+      if (L.busy || pending_.empty() || stop_) continue;
+      // beside launches in flight a young request waits for company
+      if (busy && (int)pending_.size() < kMaxJobs && now_ms() - reqs_[pending_.front()].t_submit < kCompanyMs) break;
+      progress |= launch_locked(L);
+      busy |= L.busy;
+    }
     if (stop_ && !busy) break;
     if (progress) continue;
     if (memory_wait_) {

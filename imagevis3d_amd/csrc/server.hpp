@@ -37,6 +37,11 @@ namespace tvk {
 // Estimated samples (tile-rect rays x the volume's longest axis in steps)
 // one launch may carry beyond its first request: about 5 ms of raycasting.
 constexpr uint64_t kLaunchCostCap = 1000000000ull;
+// While other launches are in flight, a request waits up to this long for
+// company before it takes a free lane.  Light requests come back in 0.1 to
+// 0.2 ms, less than a client needs to submit the next few, and would each
+// take a launch of their own.
+constexpr double kCompanyMs = 0.1;
 // Default part cost: a request of more estimated samples renders in parts of
 // at most this many (about 20 ms of raycasting each), and at most kMaxParts.
 constexpr uint64_t kPartCost = 4000000000ull;
