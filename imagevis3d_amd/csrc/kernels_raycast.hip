@@ -248,8 +248,9 @@ __device__ inline void fetch_value_grad(const T* __restrict__ base, const SlotGe
 // in LDS (render_tile_staged).
 // kModeGradGroup: the gradient march of a TF group -- one walk per ray
 // compositing up to kGroupMax TFs (render_tile_group).
+// kModeGradLone: its quad march for launches without groups.
 constexpr int kMode1D = 0, kModeGrad = 1, kModeIso = 2, kModeRegions = 3, kModeMIP = 4, kMode1DStaged = 5,
-              kModeGradGroup = 6;
+              kModeGradGroup = 6, kModeGradLone = 7;
 
 // Device address of brick gid's slot from the page table (null: the brick
 // is not resident).  Slots may live in any allocation of the device pool.
@@ -1081,12 +1082,12 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
 // brick changes (a member's own march stops rounding once it has
 // terminated), asks for a non-resident brick and touches a resident one
 // that some member needs.  Returns whether the unit has samples to gather.
-template <typename T, bool LINEAR>
-__device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* const (&Q)[kGroupMax], int F,
+template <typename T, bool LINEAR, int GM>
+__device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* const (&Q)[GM], int F,
                                   const Ray& r, const Walk& walk,
                                   int k, int n, float t0, float step, float lastlen, uint32_t live, int& kend,
                                   uint32_t& need, const T* __restrict__& base, float (&g0)[3], int& blend_gid,
-                                  float (&C)[kGroupMax][3], float (&A)[kGroupMax]) {
+                                  float (&C)[GM][3], float (&A)[GM]) {
   const LodInfo& lv = P.level;
   const float len0 = (k == n - 1) ? lastlen : step;
   const float tk = fmaf((float)k, step, t0) + 0.5f * len0;
@@ -1098,7 +1099,7 @@ __device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* c
   need = 0;
   uint32_t level = P.skip ? 15u : 0u;
 #pragma unroll
-  for (int f = 0; f < kGroupMax; ++f)
+  for (int f = 0; f < GM; ++f)
     if (f < F && (live >> f & 1u)) {
       const uint32_t code = P.skip ? gload(Q[f]->cell_code + cidx) : 0u;
       if (!(code & 1u)) need |= 1u << f;
@@ -1108,7 +1109,7 @@ __device__ inline bool group_unit(const RaycastParams& P, const RaycastParams* c
   base = brick_base<T>(P, gid);
   if (P.blend_bits < 32 && gid != blend_gid) {
 #pragma unroll
-    for (int f = 0; f < kGroupMax; ++f)
+    for (int f = 0; f < GM; ++f)
       if (live >> f & 1u) blend_round(P.blend_bits, C[f][0], C[f][1], C[f][2], A[f]);
     blend_gid = gid;
   }
@@ -1708,7 +1709,17 @@ constexpr int kQuadSubs = 4;   // quad waves per ray tile
 // quarter of the serial chain per wave and no shuffles or LDS.  Lit 720p
 // frame of a u8 scan alone 727 -> 333 us, in a row 306 -> 237; 16 lit 2D-TF
 // views of 1 GiB 24.6 -> 23.2 ms, bound by the 16 voxel and 4 texel gathers.
-template <typename T, bool LINEAR>
+//
+// GM: the most members a group of the launch has.  Launches without groups
+// (single frames, served requests) run GM = 1 (kModeGradLone), which fits 128
+// registers and so 4 waves a SIMD instead of 3 (trilinear; the nearest march
+// would spill), and there the four waves of a work-group take the quarters
+// of one tile together, a barrier per tile: a quarter of the tickets, and
+// neighbouring rays share a CU's cache.  Lit 720p frame 225 -> 198 us by GM,
+// 167 by shared tiles, 152 by registers; 24 served requests 10.4 -> 9.8 ms.
+// Groups keep a ticket per quarter: with shared tiles the 16 views of 1 GiB
+// took 22.4 ms against 21.8.
+template <typename T, bool LINEAR, int GM>
 __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, const RaycastParams& P,
                                               const float4* __restrict__ lds,
                                               int tile, int sub, int lane, uint32_t (&n_eval)[kGroupMax],
@@ -1718,14 +1729,14 @@ __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, 
   uint32_t nom = 0;
   if (!setup_ray(P, tile, sub * (64 / kQuadSubs) + lane / kQuad, r, nom)) return;
   if (q == 0) n_nom += nom;
-  const int F = P.group_n > 1 ? P.group_n : 1;
-  const RaycastParams* Q[kGroupMax];
+  const int F = GM > 1 && P.group_n > 1 ? P.group_n : 1;
+  const RaycastParams* Q[GM];
   Q[0] = &P;
 #pragma unroll
-  for (int f = 1; f < kGroupMax; ++f) Q[f] = f < F ? &tab->jobs[P.group_jobs[f - 1]] : &P;
-  float C[kGroupMax][3], A[kGroupMax];
+  for (int f = 1; f < GM; ++f) Q[f] = f < F ? &tab->jobs[P.group_jobs[f - 1]] : &P;
+  float C[GM][3], A[GM];
 #pragma unroll
-  for (int f = 0; f < kGroupMax; ++f) C[f][0] = C[f][1] = C[f][2] = A[f] = 0.f;
+  for (int f = 0; f < GM; ++f) C[f][0] = C[f][1] = C[f][2] = A[f] = 0.f;
   const float t0 = r.t0, L = r.t1 - r.t0;
   if (r.hit && L > 0.f) {
     const float step = P.step;
@@ -1781,7 +1792,7 @@ __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, 
       const float gm = sqrtf(g[0] * g[0] + g[1] * g[1] + g[2] * g[2]);
       uint32_t most = 0;  // samples of the four that some member evaluates
 #pragma unroll
-      for (int f = 0; f < kGroupMax; ++f) {
+      for (int f = 0; f < GM; ++f) {
         if (!(need >> f & 1u)) continue;
         float cs[4];
         tf_lookup(*Q[f], lds, v, gm, cs);
@@ -1807,11 +1818,11 @@ __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, 
     }
     if (P.blend_bits < 32)
 #pragma unroll
-      for (int f = 0; f < kGroupMax; ++f) blend_round(P.blend_bits, C[f][0], C[f][1], C[f][2], A[f]);
+      for (int f = 0; f < GM; ++f) blend_round(P.blend_bits, C[f][0], C[f][1], C[f][2], A[f]);
   }
   const int64_t pix = (int64_t)r.py * P.width + r.px;
 #pragma unroll
-  for (int f = 0; f < kGroupMax; ++f)
+  for (int f = 0; f < GM; ++f)
     if (f < F && q == (f & (kQuad - 1)))
       gstore(Q[f]->framebuffer + pix, over_background(P, r.py, C[f][0], C[f][1], C[f][2], A[f]));
 }
@@ -1820,12 +1831,12 @@ __device__ inline void render_tile_group_quad(const JobTable* __restrict__ tab, 
 // taken from the per-XCD queues until all queues are drained.  Tile t of
 // the launch belongs to job j with tile_start[j] <= t < tile_start[j + 1].
 template <typename T, bool LINEAR, int BATCH, bool TF_LDS, int MODE>
-__global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __restrict__ tab) {
+__global__ __launch_bounds__(kThreads, MODE == kModeGradLone && LINEAR ? 4 : 2) void raycast_kernel(const JobTable* __restrict__ tab) {
   const int kT = (int)blockDim.x;  // 256 or 512 threads (see launch_one)
   // TF_LDS: the launch's 1D TF, n_tf_lds + 1 entries; gradient launches
   // without it: the tables the host chose
   extern __shared__ float4 s_tf[];
-  constexpr bool kGradTables = !TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup);
+  constexpr bool kGradTables = !TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup || MODE == kModeGradLone);
   __shared__ unsigned long long s_count[kJobCounters * kMaxJobs];  // per job: evaluated, nominal, gathered
   const JobTableHeader& H = tab->h;
   const float4* tf_shared = (const float4*)H.tf_lds;
@@ -1847,7 +1858,8 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
   const int total = H.total_tiles;
   const int G = H.tile_group;
   // quad waves take a quarter of a ray tile per ticket
-  constexpr int kSubShift = (MODE == kModeGradGroup && BATCH == kQuad) ? 2 : 0;
+  constexpr bool kShared = MODE == kModeGradLone;
+  constexpr int kSubShift = !kShared && ((MODE == kModeGradGroup && BATCH == kQuad) || MODE == kModeGradLone) ? 2 : 0;
   static_assert(1 << 2 == kQuadSubs, "a quad ticket is tile * kQuadSubs + quarter");
   // xcd_split regions apply to one-job launches only
   const int split = n_jobs == 1 ? H.xcd_split : 0;
@@ -1862,7 +1874,7 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
   // adds the wave's counts of cur_job (and of its group's members) to the
   // work-group's counters
   auto flush = [&]() {
-    if constexpr (MODE == kModeGradGroup) {
+    if constexpr (MODE == kModeGradGroup || MODE == kModeGradLone) {
       const RaycastParams& Pc = tab->jobs[cur_job];
       const int F = Pc.group_n > 1 ? Pc.group_n : 1;
 #pragma unroll
@@ -1901,69 +1913,103 @@ __global__ __launch_bounds__(kThreads, 2) void raycast_kernel(const JobTable* __
     return rw * rh;
   };
   int x = xcd;  // own queue first, then steal
-  while (true) {
-    int rx0, rw, ry0;
-    const int slots = region(x, rx0, rw, ry0);
+  // The next ticket: its tile, and `at` the ticket itself, or -1 once every
+  // queue is drained.
+  auto next = [&](int& at) -> int {
     while (true) {
-      // Every lane takes part in the queue atomic (lanes other than 0 add
-      // 0; the compiler reduces it to one atomic per wave) and all branches
-      // in this loop are wave-uniform: no lane-0-only block in the source
-      // that the compiler could split off the loop around the wave-wide
-      // broadcast of the ticket.
-      const unsigned long long ticket = wave_atomic_add(&queues[x * kQueueStride], lane == 0 ? 1ull : 0ull);
-      const int at = __builtin_amdgcn_readfirstlane((int)__shfl((long long)ticket, 0, 64));
-      const int pos = at >> kSubShift;
-      if (pos >= slots) break;
-      int tile;
-      if (split == 0) tile = ((pos / G) * 8 + x) * G + (pos % G);
-      else tile = (ry0 + pos / rw) * tiles_x0 + rx0 + pos % rw;
-      if (tile >= total) continue;
-      // the job of this tile (wave-uniform binary search over the prefix)
-      int lo = 0, hi = n_jobs - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (tab->tile_start[mid] <= tile) lo = mid;
-        else hi = mid - 1;
+      int rx0, rw, ry0;
+      const int slots = region(x, rx0, rw, ry0);
+      while (true) {
+        // Every lane takes part in the queue atomic (lanes other than 0 add
+        // 0; the compiler reduces it to one atomic per wave) and all
+        // branches in this loop are wave-uniform: no lane-0-only block in
+        // the source that the compiler could split off the loop around the
+        // wave-wide broadcast of the ticket.
+        const unsigned long long ticket = wave_atomic_add(&queues[x * kQueueStride], lane == 0 ? 1ull : 0ull);
+        at = __builtin_amdgcn_readfirstlane((int)__shfl((long long)ticket, 0, 64));
+        const int pos = at >> kSubShift;
+        if (pos >= slots) break;
+        int tile;
+        if (split == 0) tile = ((pos / G) * 8 + x) * G + (pos % G);
+        else tile = (ry0 + pos / rw) * tiles_x0 + rx0 + pos % rw;
+        if (tile < total) return tile;
       }
-      const int job = __builtin_amdgcn_readfirstlane(lo);
-      const RaycastParams& P = tab->jobs[job];
-      const float4* tf4 = TF_LDS ? tf_shared : (const float4*)P.tf;
-      if (job != cur_job) {  // wave-uniform
-        if (cur_job >= 0) flush();
-        cur_job = job;
-        n_eval = n_nom = 0;
-      }
-      // the job's own tile slot (a part's slots start at tile_first)
-      const int slot = tile - tab->tile_start[job] + P.tile_first;
-      if constexpr (MODE == kMode1DStaged) {
-        // this wave's staging buffer follows the LDS TF
-        T* sbuf = (T*)(s_tf + (TF_LDS ? H.n_tf_lds + 1 : 0)) + (threadIdx.x >> 6) * kStageElems;
-        render_tile_staged<T, TF_LDS>(P, tf4, slot, lane, n_eval, n_nom, sbuf);
-      } else if constexpr (MODE == kModeGradGroup && BATCH == kQuad) {
-        render_tile_group_quad<T, LINEAR>(tab, P, s_tf, slot, at & (kQuadSubs - 1), lane, n_evalg, n_walk, n_nom);
-      } else if constexpr (MODE == kModeGradGroup) {
-        render_tile_group<T, LINEAR, BATCH>(tab, P, s_tf, slot, lane, n_evalg, n_walk, n_nom);
-      } else {
-        render_tile<T, LINEAR, BATCH, MODE, TF_LDS>(P, tf4, s_tf, slot, lane, n_eval, n_nom);
-      }
+      // This queue is drained: one load per lane looks at all heads, and the
+      // wave goes on at the next queue that still has tiles.  Heads only
+      // grow, and a wave that finds a queue drained after all looks again, so
+      // the loop ends once every head has passed its slots.  (A failing
+      // ticket on each of the other queues instead cost every wave 7
+      // atomics: 16,000 for 2048 waves, 0.17 ms of any launch.  A 512x512
+      // capture of 64^3 u8 407 -> 238 us, a 1080p isosurface frame of 512^3
+      // u16 369 -> 258, a lit 720p frame 445 -> 350.)
+      const int qx = lane & 7;
+      int ux0, uw, uy0;
+      const int qslots = region(qx, ux0, uw, uy0);
+      const unsigned long long head = __hip_atomic_load((global_u64*)&queues[qx * kQueueStride], __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+      const uint32_t open = (uint32_t)(__ballot(head < (unsigned long long)qslots << kSubShift) & 0xffull);
+      if (open == 0) return -1;
+      const uint32_t ahead = ((open | open << 8) >> x) & 0xffu;  // bit k: queue (x + k) & 7 has tiles
+      x = (x + __builtin_ctz(ahead)) & 7;
     }
-    // This queue is drained: one load per lane looks at all heads, and the
-    // wave goes on at the next queue that still has tiles.  Heads only
-    // grow, and a wave that finds a queue drained after all looks again, so
-    // the loop ends once every head has passed its slots.  (A failing
-    // ticket on each of the other queues instead cost every wave 7
-    // atomics: 16,000 for 2048 waves, 0.17 ms of any launch.  A 512x512
-    // capture of 64^3 u8 407 -> 238 us, a 1080p isosurface frame of 512^3
-    // u16 369 -> 258, a lit 720p frame 445 -> 350.)
-    const int qx = lane & 7;
-    int ux0, uw, uy0;
-    const int qslots = region(qx, ux0, uw, uy0);
-    const unsigned long long head = __hip_atomic_load((global_u64*)&queues[qx * kQueueStride], __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t open = (uint32_t)(__ballot(head < (unsigned long long)qslots << kSubShift) & 0xffull);
-    if (open == 0) break;
-    const uint32_t ahead = ((open | open << 8) >> x) & 0xffu;  // bit k: queue (x + k) & 7 has tiles
-    x = (x + __builtin_ctz(ahead)) & 7;
+  };
+  auto render = [&](int tile, int sub) {
+    // the job of this tile (wave-uniform binary search over the prefix)
+    int lo = 0, hi = n_jobs - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (tab->tile_start[mid] <= tile) lo = mid;
+      else hi = mid - 1;
+    }
+    const int job = __builtin_amdgcn_readfirstlane(lo);
+    const RaycastParams& P = tab->jobs[job];
+    const float4* tf4 = TF_LDS ? tf_shared : (const float4*)P.tf;
+    if (job != cur_job) {  // wave-uniform
+      if (cur_job >= 0) flush();
+      cur_job = job;
+      n_eval = n_nom = 0;
+    }
+    // the job's own tile slot (a part's slots start at tile_first)
+    const int slot = tile - tab->tile_start[job] + P.tile_first;
+    if constexpr (MODE == kMode1DStaged) {
+      // this wave's staging buffer follows the LDS TF
+      T* sbuf = (T*)(s_tf + (TF_LDS ? H.n_tf_lds + 1 : 0)) + (threadIdx.x >> 6) * kStageElems;
+      render_tile_staged<T, TF_LDS>(P, tf4, slot, lane, n_eval, n_nom, sbuf);
+    } else if constexpr (MODE == kModeGradLone) {
+      render_tile_group_quad<T, LINEAR, 1>(tab, P, s_tf, slot, sub, lane, n_evalg, n_walk, n_nom);
+    } else if constexpr (MODE == kModeGradGroup && BATCH == kQuad) {
+      render_tile_group_quad<T, LINEAR, kGroupMax>(tab, P, s_tf, slot, sub, lane, n_evalg, n_walk,
+                                                   n_nom);
+    } else if constexpr (MODE == kModeGradGroup) {
+      render_tile_group<T, LINEAR, BATCH>(tab, P, s_tf, slot, lane, n_evalg, n_walk, n_nom);
+    } else {
+      render_tile<T, LINEAR, BATCH, MODE, TF_LDS>(P, tf4, s_tf, slot, lane, n_eval, n_nom);
+    }
+  };
+  if constexpr (kShared) {
+    // Each kQuadSubs waves of the work-group take a tile together, a quarter
+    // each; the first waves take the tickets.
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int tiles = kT / 64 / kQuadSubs;
+    __shared__ int s_tile[2][kWaves / kQuadSubs];
+    for (int turn = 0;; turn ^= 1) {
+      if (wave < tiles) {
+        int at;
+        const int t = next(at);
+        s_tile[turn][wave] = t;
+      }
+      // s_tile[turn] is written again only after the next turn's barrier,
+      // which every wave reaches after it has read this turn's
+      __syncthreads();
+      bool any = false;
+      for (int w = 0; w < tiles; ++w) any |= s_tile[turn][w] >= 0;
+      if (!__builtin_amdgcn_readfirstlane((int)any)) break;  // the same for every wave
+      const int t = __builtin_amdgcn_readfirstlane(s_tile[turn][wave / kQuadSubs]);
+      if (t >= 0) render(t, wave % kQuadSubs);
+    }
+  } else {
+    int at;
+    for (int t = next(at); t >= 0; t = next(at)) render(t, at & (kQuadSubs - 1));
   }
   if (cur_job >= 0) flush();
   __syncthreads();
@@ -1984,7 +2030,7 @@ hipError_t launch_one(const LaunchInfo& li, const JobTable* tab, hipStream_t str
   // which is faster on cache-friendly volumes and slower where more waves
   // in flight thrash the caches (the autotuner picks).
   const int kT = TF_LDS ? kThreads : 64 * (li.wg_waves == 4 ? 4 : 8);
-  if (!TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup)) lds += (size_t)li.lds_quads * sizeof(float4);
+  if (!TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup || MODE == kModeGradLone)) lds += (size_t)li.lds_quads * sizeof(float4);
   if (MODE == kMode1DStaged) lds += (size_t)(kT / 64) * kStageElems * sizeof(T);  // per-wave cell buffers
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kT, lds);
   if (e != hipSuccess) return e;
@@ -2019,7 +2065,8 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
   if (li.mode == 1 || li.lighting) {
     if (li.batch == 1) return launch_grad<T, LINEAR, 1>(li, tab, stream);
     if (li.batch == 2) return launch_grad<T, LINEAR, 2>(li, tab, stream);
-    return launch_one<T, LINEAR, kQuad, false, kModeGradGroup>(li, tab, stream);
+    return li.group ? launch_one<T, LINEAR, kQuad, false, kModeGradGroup>(li, tab, stream)
+                    : launch_one<T, LINEAR, kQuad, false, kModeGradLone>(li, tab, stream);
   }
   const bool lds = li.n_tf_lds > 0;
   if (li.stage && LINEAR && !li.lighting)
