@@ -493,6 +493,7 @@ void MemMan::ParallelFor(size_t n, int threads, const std::function<void(size_t)
     return;
   }
   std::lock_guard<std::mutex> pg(par_mu_);
+  par_busy_ = true;
   {
     std::lock_guard<std::mutex> lk(wmu_);
     while ((int)workers_.size() < threads - 1) workers_.emplace_back([this] { worker(); });
@@ -508,6 +509,13 @@ void MemMan::ParallelFor(size_t n, int threads, const std::function<void(size_t)
   std::unique_lock<std::mutex> lk(wmu_);
   wdone_.wait(lk, [&] { return job_active_ == 0; });
   job_ = nullptr;
+  par_busy_ = false;
+}
+
+bool MemMan::TryParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn) {
+  if (par_busy_) return false;  // always seen by a call from inside fn
+  ParallelFor(n, threads, fn);
+  return true;
 }
 
 }  // namespace tvk

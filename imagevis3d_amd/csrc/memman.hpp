@@ -110,6 +110,10 @@ class MemMan {
   // Runs fn(0..n) on up to `threads` workers (the caller works too) and
   // returns when all are done.
   void ParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn);
+  // The same, unless the workers are busy: returns false and runs nothing.
+  // For work that may itself run inside fn (a brick source that reads
+  // another renderer's frame), where waiting for the workers would never end.
+  bool TryParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn);
 
  private:
   explicit MemMan(int device);
@@ -178,6 +182,7 @@ class MemMan {
   uint64_t job_gen_ = 0;
   bool stop_ = false;
   std::mutex par_mu_;  // one ParallelFor at a time
+  std::atomic<bool> par_busy_{false};  // one is running
 };
 
 }  // namespace tvk

@@ -253,6 +253,7 @@ HipRenderer::~HipRenderer() {
     cell_range_.reset();
     framebuffer_.reset();
     lowres_fb_.reset();
+    pipe_.Release();
     if (copy_stream_) (void)hipStreamDestroy(copy_stream_);
     if (stream_) (void)hipStreamDestroy(stream_);
   }
@@ -462,7 +463,7 @@ int HipRenderer::set_volume_impl(const void* voxels, int gen_kind, uint64_t seed
 
   for (int l = 0; l < nl; ++l) TVK_HIP(levels_[l].alloc(ld[l][0] * ld[l][1] * ld[l][2] * bpv));
   if (voxels) {
-    TVK_HIP(hipMemcpyAsync(levels_[0].p, voxels, levels_[0].bytes, hipMemcpyHostToDevice, stream_));
+    TVK_HIP(pipe_.Upload(device_, levels_[0].p, voxels, levels_[0].bytes, stream_));
   } else {
     const int64_t d[3] = {(int64_t)dims[0], (int64_t)dims[1], (int64_t)dims[2]};
     const int64_t slab = std::max<int64_t>(1, (int64_t)((1ull << 30) / (dims[0] * dims[1])));
@@ -679,9 +680,8 @@ int HipRenderer::ReadRegionOutput(int32_t* out, uint64_t n) {
   if (!region_out_on_ || !region_out_dev_.p) return state_fail("region output is off (or nothing painted)");
   if (!out || n < (uint64_t)width_ * height_) return arg_fail("region output buffer too small");
   TVK_HIP(hipSetDevice(device_));
-  TVK_HIP(hipMemcpyAsync(out, region_out_dev_.p, (size_t)width_ * height_ * 4, hipMemcpyDeviceToHost,
-                         stream_));
-  TVK_HIP(hipStreamSynchronize(stream_));
+  const CopyPiece piece{out, region_out_dev_.p, (size_t)width_ * height_ * 4};
+  TVK_HIP(pipe_.Download(device_, &piece, 1, stream_));
   return TVK_OK;
 }
 
@@ -808,8 +808,8 @@ int HipRenderer::ReadLod(uint32_t lod, void* out, uint64_t bytes) {
   }
   if (!out || bytes < levels_[lod].bytes) return arg_fail("output buffer too small");
   TVK_HIP(hipSetDevice(device_));
-  TVK_HIP(hipMemcpyAsync(out, levels_[lod].p, levels_[lod].bytes, hipMemcpyDeviceToHost, stream_));
-  TVK_HIP(hipStreamSynchronize(stream_));
+  const CopyPiece piece{out, levels_[lod].p, levels_[lod].bytes};
+  TVK_HIP(pipe_.Download(device_, &piece, 1, stream_));
   return TVK_OK;
 }
 
@@ -1340,8 +1340,8 @@ int HipRenderer::ReadFramebuffer(uint8_t* rgba, uint64_t bytes) {
   if (!rgba || bytes < (uint64_t)width_ * height_ * 4) return arg_fail("framebuffer readback buffer too small");
   if (int e = resolve_check()) return e;
   TVK_HIP(hipSetDevice(device_));
-  TVK_HIP(hipMemcpyAsync(rgba, framebuffer_.p, (size_t)width_ * height_ * 4, hipMemcpyDeviceToHost, stream_));
-  TVK_HIP(hipStreamSynchronize(stream_));
+  const CopyPiece piece{rgba, framebuffer_.p, (size_t)width_ * height_ * 4};
+  TVK_HIP(pipe_.Download(device_, &piece, 1, stream_));
   return TVK_OK;
 }
 
@@ -2028,6 +2028,7 @@ int HipRenderer::RenderBatch(const tvk_view* views, uint32_t n, tvk_view_stats* 
   const int lo = std::min<int>((int)lod_min_, n_lod_ - 1);
   const int hi = std::max(lo, std::min<int>((int)lod_max_, n_lod_ - 1));
   float kms = 0.f;
+  std::vector<CopyPiece> images;  // the views to copy out
   for (uint32_t first = 0; first < n; first += kMaxJobs) {
     const int cnt = (int)std::min<uint32_t>(kMaxJobs, n - first);
     // one shared 1D TF goes to LDS
@@ -2106,11 +2107,11 @@ int HipRenderer::RenderBatch(const tvk_view* views, uint32_t n, tvk_view_stats* 
         stats[i].reserved = 0;
       }
       if (views[i].rgba)
-        TVK_HIP(hipMemcpyAsync(views[i].rgba, (uint8_t*)batch_fb_.p + batch_fb_offset_[i],
-                               (size_t)views[i].width * views[i].height * 4, hipMemcpyDeviceToHost,
-                               stream_));
+        images.push_back(CopyPiece{views[i].rgba, (uint8_t*)batch_fb_.p + batch_fb_offset_[i],
+                                   (size_t)views[i].width * views[i].height * 4});
     }
-    TVK_HIP(hipStreamSynchronize(stream_));
+    TVK_HIP(pipe_.Download(device_, images.data(), images.size(), stream_));
+    images.clear();
   }
   if (kernel_ms) *kernel_ms = kms;
   return TVK_OK;
@@ -2311,9 +2312,8 @@ int HipRenderer::Capture(uint8_t* rgba, uint64_t bytes, bool preserve) {
   }
   if (rc == TVK_OK) rc = resolve_check();
   if (rc == TVK_OK) {
-    hipError_t e = hipMemcpyAsync(rgba, framebuffer_.p, (size_t)width_ * height_ * 4,
-                                  hipMemcpyDeviceToHost, stream_);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream_);
+    const CopyPiece piece{rgba, framebuffer_.p, (size_t)width_ * height_ * 4};
+    const hipError_t e = pipe_.Download(device_, &piece, 1, stream_);
     if (e != hipSuccess) rc = hip_fail(e, "capture readback");
   }
   if (preserve) {

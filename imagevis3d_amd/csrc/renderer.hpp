@@ -17,6 +17,7 @@
 #include "../../include/tvk_hip.h"
 #include "kernels.hpp"
 #include "memman.hpp"
+#include "transfer.hpp"
 #include "tvk_common.hpp"
 
 namespace tvk {
@@ -449,6 +450,7 @@ class HipRenderer : public PoolClient {
   int staging_round_ = 0;              // bricks per round
   uint64_t staging_host_bytes_ = 0;    // accounted as host memory
   hipStream_t copy_stream_ = nullptr;  // brick uploads
+  HostPipe pipe_;  // large copies between caller memory and stream_
   hipEvent_t upload_done_ = nullptr;
   int pool_client_ = -1;               // MemMan client id of a paged volume
   std::mutex pool_mu_;                 // page table vs evictions from other threads

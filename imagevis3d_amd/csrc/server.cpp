@@ -528,7 +528,7 @@ int RenderServer::Wait(uint64_t ticket, uint32_t timeout_ms, tvk_request_result*
   const bool copy = r.status == TVK_OK && r.q.view.rgba;
   lk.unlock();
   // the host block stays reserved until the copy into the caller's buffer
-  if (copy) memcpy(r.q.view.rgba, host_arena_mem_ + r.host_off, r.bytes);
+  if (copy) parallel_memcpy(device_, r.q.view.rgba, host_arena_mem_ + r.host_off, r.bytes);
   if (r.host_held) {
     std::lock_guard<std::mutex> g(mu_);
     host_arena_.free(r.host_off, r.bytes);
