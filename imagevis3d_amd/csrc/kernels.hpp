@@ -14,15 +14,18 @@ namespace tvk {
 hipError_t launch_downsample(const void* src, int bpv, const int64_t src_dims[3], void* dst,
                              hipStream_t stream, bool median = false);
 
+// u32 words of `scratch` that launch_extract_bricks needs for n_jobs bricks of
+// slot edge S.
+int64_t extract_scratch_words(int64_t n_jobs, int S);
 // Cut `n_jobs` bricks of payload B with apron a out of a flat level into
 // pool slots (blocked slot layout, clamp-to-edge outside the volume) and
 // write each brick's (min, max) over the slot to brick_range[2*brick_id].
-// Slot j starts at element j * slot_stride of the pool; scratch_minmax
-// holds 2 u32 per job.
+// Slot j starts at element j * slot_stride of the pool; scratch holds
+// extract_scratch_words(n_jobs, B + 2a) u32.
 hipError_t launch_extract_bricks(const void* level, int bpv, const int64_t dims[3],
                                  const BrickJob* jobs, int n_jobs, void* pool,
                                  int64_t slot_stride, int B, int apron, float* brick_range,
-                                 uint32_t* scratch_minmax, hipStream_t stream);
+                                 uint32_t* scratch, hipStream_t stream);
 
 // Overlap-inclusive x-fastest bricks (S = P + 2o per axis) of a flat level
 // for the TOC builder: job j (its `slot` field = index into `out` and into

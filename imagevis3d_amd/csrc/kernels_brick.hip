@@ -80,6 +80,19 @@ __global__ __launch_bounds__(kThreads) void downsample_kernel(const T* __restric
   }
 }
 
+// N consecutive voxels with one load; a volume row starts at any multiple of
+// the voxel size, and unaligned global loads are legal on gfx950.
+template <typename T, int N>
+struct VoxelRun {
+  typedef T vec __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+};
+template <typename T, int N>
+__device__ inline void load_run(const T* p, uint32_t (&out)[N]) {
+  const auto v = *(const __attribute__((address_space(1))) typename VoxelRun<T, N>::vec*)p;
+#pragma unroll
+  for (int j = 0; j < N; ++j) out[j] = v[j];
+}
+
 __device__ inline uint32_t wave_min(uint32_t v) {
   for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o, 64));
   return v;
@@ -100,51 +113,119 @@ __device__ inline int64_t clamp64(int64_t v, int64_t lo, int64_t hi) {
   return v < lo ? lo : (v > hi ? hi : v);
 }
 
-// Slot-local voxel of element i of a slot in the blocked slot layout
-// (tvk_common.hpp); the overlap voxel past a block row's end and padding
-// past the slot's edge repeat the slot's last voxel along that axis.
-__device__ inline void slot_element_voxel(uint32_t i, int S, int& x, int& y, int& z) {
-  const uint32_t n = (uint32_t)slot_blocks(S);
-  const uint32_t b = i / kSlotBlockElems, r = i % kSlotBlockElems;
-  const uint32_t row = r / 5, e = r % 5;
-  x = min((int)((b % n) * 4 + e), S - 1);
-  y = min((int)(((b / n) % n) * 4 + (row & 3)), S - 1);
-  z = min((int)((b / (n * n)) * 4 + (row >> 2)), S - 1);
+// One row of a slot's blocks (all bx at by, bz) in the blocked slot layout:
+// the 16 rows of x its blocks hold come in as contiguous runs, wait in LDS
+// and leave in element order -- the row's blocks are contiguous in the slot
+// -- 16 bytes a thread and step.  The slot's voxel (x, y, z) is src at (ox +
+// x, oy + y, oz + z) clamped to the nx x ny x nz volume; blocks past the
+// slot's edge repeat its last voxel along that axis.  lds: 16 rows of 4 (n +
+// 1) voxels.  Folds the voxels' range into lo and hi.
+template <typename T>
+__device__ inline void slot_block_row(const T* __restrict__ src, int64_t nx, int64_t ny, int64_t nz, int64_t ox,
+                                      int64_t oy, int64_t oz, int S, int by, int bz, T* __restrict__ slot, T* lds,
+                                      uint32_t& lo, uint32_t& hi) {
+  const int n = slot_blocks(S), segs = n + 1, stride = 4 * segs;
+  const int row = (int)threadIdx.x >> 4;  // 16 rows, 16 threads each
+  const int64_t y = clamp64(oy + min(by * 4 + (row & 3), S - 1), 0, ny - 1);
+  const int64_t z = clamp64(oz + min(bz * 4 + (row >> 2), S - 1), 0, nz - 1);
+  const T* __restrict__ line = src + (z * ny + y) * nx;
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  for (int seg = (int)threadIdx.x & 15; seg < segs; seg += 16) {
+    const int x = 4 * seg;
+    const int64_t gx = ox + x;
+    uint32_t v[4];
+    if (x + 3 < S && gx >= 0 && gx + 3 < nx) {
+      load_run<T, 4>(line + gx, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = line[clamp64(ox + min(x + j, S - 1), 0, nx - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lo = min(lo, v[j]);
+      hi = max(hi, v[j]);
+    }
+    *(vec4*)(lds + row * stride + x) = vec4{(T)v[0], (T)v[1], (T)v[2], (T)v[3]};
+  }
+  __syncthreads();
+  constexpr int N = 16 / (int)sizeof(T);  // a block's 80 voxels are a multiple of it
+  T* __restrict__ out = slot + (int64_t)(bz * n + by) * n * kSlotBlockElems;
+  for (int g = (int)threadIdx.x; g < n * (kSlotBlockElems / N); g += kThreads) {
+    const uint32_t i = (uint32_t)g * N, bx = i / kSlotBlockElems, r = i % kSlotBlockElems;
+    const T* q = lds + (r / 5) * stride + bx * 4;
+    int e = (int)(r % 5);
+    T v[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      v[j] = q[e];
+      if (++e == 5) {
+        e = 0;
+        q += stride;
+      }
+    }
+    uint4 w;
+    __builtin_memcpy(&w, v, sizeof w);
+    *(uint4*)(out + i) = w;
+  }
 }
 
-// grid.x: chunks of one slot, grid.y: brick job.  Writes the slot in
-// element order (coalesced), reading the level voxel each element holds.
+// Bricks of a flat level into pool slots.  grid.y: brick job; work-group p of
+// grid.x takes the slot's block rows [p per, (p + 1) per) (row by + bz n) and
+// leaves their range in part[2 (job gridDim.x + p)].  HBM stream: the level
+// once (aprons from the caches), the slots once.  An element per thread and
+// step (five divisions, a 2-byte load and store) and two atomics a wave on
+// its brick's range took 1.17 ms for the 64 bricks of 128^3 of a 512^3 u16
+// level and 3.9 ms for the 512 of 1024^3 u8; 0.18 and 1.2 now.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void extract_bricks_kernel(
     const T* __restrict__ level, int64_t nx, int64_t ny, int64_t nz,
-    const BrickJob* __restrict__ jobs, T* __restrict__ pool, int64_t slot_stride, int64_t slot_elems,
-    int B, int apron, uint32_t* __restrict__ minmax) {
+    const BrickJob* __restrict__ jobs, T* __restrict__ pool, int64_t slot_stride,
+    int B, int apron, int per, uint32_t* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __shared__ uint32_t s_lo[kThreads / 64], s_hi[kThreads / 64];
   const BrickJob job = jobs[blockIdx.y];
-  const int S = B + 2 * apron;
-  const int64_t ox = (int64_t)job.bx * B - apron;
-  const int64_t oy = (int64_t)job.by * B - apron;
-  const int64_t oz = (int64_t)job.bz * B - apron;
-  T* __restrict__ slot = pool + job.slot * slot_stride;
-  const int64_t chunk = (slot_elems + gridDim.x - 1) / gridDim.x;
-  const int64_t beg = chunk * blockIdx.x;
-  const int64_t end = beg + chunk < slot_elems ? beg + chunk : slot_elems;
+  const int S = B + 2 * apron, n = slot_blocks(S);
   uint32_t lo = 0xffffffffu, hi = 0;
-  for (int64_t i = beg + threadIdx.x; i < end; i += kThreads) {
-    int x, y, z;
-    slot_element_voxel((uint32_t)i, S, x, y, z);  // slot_elems < 2^31 (checked by the host)
-    const int64_t gx = clamp64(ox + x, 0, nx - 1);
-    const int64_t gy = clamp64(oy + y, 0, ny - 1);
-    const int64_t gz = clamp64(oz + z, 0, nz - 1);
-    const T v = level[(gz * ny + gy) * nx + gx];
-    slot[i] = v;
-    lo = min(lo, (uint32_t)v);
-    hi = max(hi, (uint32_t)v);
+  const int r0 = (int)blockIdx.x * per, r1 = min(r0 + per, n * n);
+  for (int r = r0; r < r1; ++r) {
+    if (r > r0) __syncthreads();  // the last row's voxels have been written out
+    slot_block_row<T>(level, nx, ny, nz, (int64_t)job.bx * B - apron, (int64_t)job.by * B - apron,
+                      (int64_t)job.bz * B - apron, S, r % n, r / n, pool + job.slot * slot_stride, (T*)lds, lo, hi);
   }
   lo = wave_min(lo);
   hi = wave_max(hi);
+  const int wave = (int)(threadIdx.x >> 6);
   if ((threadIdx.x & 63) == 0) {
-    atomicMin(&minmax[2 * blockIdx.y], lo);
-    atomicMax(&minmax[2 * blockIdx.y + 1], hi);
+    s_lo[wave] = lo;
+    s_hi[wave] = hi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < kThreads / 64; ++k) {
+      lo = min(lo, s_lo[k]);
+      hi = max(hi, s_hi[k]);
+    }
+    const int64_t q = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    part[2 * q] = lo;
+    part[2 * q + 1] = hi;
+  }
+}
+
+// The bricks' ranges from their parts' (a work-group of one wave per brick).
+__global__ __launch_bounds__(64) void brick_range_kernel(const uint32_t* __restrict__ part, int parts,
+                                                         const BrickJob* __restrict__ jobs,
+                                                         float* __restrict__ brick_range) {
+  const int64_t i = blockIdx.x;
+  uint32_t lo = 0xffffffffu, hi = 0;
+  for (int k = (int)threadIdx.x; k < parts; k += 64) {
+    lo = min(lo, part[2 * (i * parts + k)]);
+    hi = max(hi, part[2 * (i * parts + k) + 1]);
+  }
+  lo = wave_min(lo);
+  hi = wave_max(hi);
+  if (threadIdx.x == 0) {
+    brick_range[2 * jobs[i].brick_id] = (float)lo;
+    brick_range[2 * jobs[i].brick_id + 1] = (float)hi;
   }
 }
 
@@ -189,16 +270,15 @@ __global__ __launch_bounds__(kThreads) void extract_linear_bricks_kernel(
   }
 }
 
-// An x-fastest S^3 brick into the blocked slot layout, and back.
+// An x-fastest S^3 brick into the blocked slot layout (grid.x: block rows),
+// and back.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void linear_to_slot_kernel(const T* __restrict__ src,
-                                                                  T* __restrict__ slot, int S,
-                                                                  int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= n) return;
-  int x, y, z;
-  slot_element_voxel((uint32_t)i, S, x, y, z);
-  slot[i] = src[((int64_t)z * S + y) * S + x];
+                                                                  T* __restrict__ slot, int S) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int n = slot_blocks(S);
+  uint32_t lo = 0xffffffffu, hi = 0;
+  slot_block_row<T>(src, S, S, S, 0, 0, 0, S, (int)blockIdx.x % n, (int)blockIdx.x / n, slot, (T*)lds, lo, hi);
 }
 
 template <typename T>
@@ -209,6 +289,65 @@ __global__ __launch_bounds__(kThreads) void slot_to_linear_kernel(const T* __res
   if (i >= n) return;
   const int x = (int)(i % S), y = (int)((i / S) % S), z = (int)(i / ((int64_t)S * S));
   dst[i] = slot[slot_offset(slot_geo(S), x, y, z)];
+}
+
+// Small empty-space cells (4 <= C <= 32, the default 16 among them): a
+// work-group owns the kx = 64 / C cells of a run along x, 64 voxels or a
+// cache line of u16, a lane a row of one of them -- neighbouring lanes the
+// neighbouring cells of a row -- and writes their packed ranges itself: no
+// clearing, global atomics or packing pass.  The voxels [c*C - 1, (c+1)*C]
+// (clamped) of a row come as runs of 4.  HBM stream of the level, read about
+// twice from the caches (18^3 voxels for 16^3 cells).  512^3 u16 in 16^3
+// cells: 0.43 ms a wave per rows of one cell, folded by atomics, 0.17 now.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void cell_range_small_kernel(const T* __restrict__ level, int64_t nx,
+                                                                    int64_t ny, int64_t nz, int C, int ncx,
+                                                                    int ncy, int64_t n_groups, int gx,
+                                                                    uint32_t* __restrict__ out) {
+  __shared__ uint32_t s_lo[16], s_hi[16];  // kx <= 16
+  const int kx = 64 / C;
+  const int k = (int)threadIdx.x % kx, lrow = (int)threadIdx.x / kx, rstep = kThreads / kx;
+  // the loop bound depends on blockIdx only: every thread reaches the barriers
+  for (int64_t g = blockIdx.x; g < n_groups; g += gridDim.x) {
+    if (threadIdx.x < 16) {
+      s_lo[threadIdx.x] = 0xffffffffu;
+      s_hi[threadIdx.x] = 0u;
+    }
+    __syncthreads();
+    const int cx = (int)(g % gx) * kx + k, cy = (int)(g / gx % ncy), cz = (int)(g / ((int64_t)gx * ncy));
+    const int64_t x0 = max((int64_t)cx * C - 1, (int64_t)0), x1 = min((int64_t)(cx + 1) * C, nx - 1);
+    const int64_t y0 = max((int64_t)cy * C - 1, (int64_t)0), y1 = min((int64_t)(cy + 1) * C, ny - 1);
+    const int64_t z0 = max((int64_t)cz * C - 1, (int64_t)0), z1 = min((int64_t)(cz + 1) * C, nz - 1);
+    const int h = (int)(y1 - y0 + 1), rows = h * (int)(z1 - z0 + 1), w = (int)(x1 - x0 + 1);
+    uint32_t lo = 0xffffffffu, hi = 0;
+    if (cx < ncx && lrow < rstep) {
+      for (int r = lrow; r < rows; r += rstep) {
+        const T* row = level + ((z0 + r / h) * ny + (y0 + r % h)) * nx + x0;
+        int x = 0;
+        for (; x + 4 <= w; x += 4) {
+          uint32_t v[4];
+          load_run<T, 4>(row + x, v);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            lo = min(lo, v[j]);
+            hi = max(hi, v[j]);
+          }
+        }
+        for (; x < w; ++x) {
+          lo = min(lo, (uint32_t)row[x]);
+          hi = max(hi, (uint32_t)row[x]);
+        }
+      }
+    }
+    if (hi >= lo) {
+      atomicMin(&s_lo[k], lo);
+      atomicMax(&s_hi[k], hi);
+    }
+    __syncthreads();
+    if (threadIdx.x < (unsigned)kx && cx < ncx)  // thread k of the first kx is cell k's
+      out[((int64_t)cz * ncy + cy) * ncx + cx] = s_lo[k] | s_hi[k] << 16;
+    __syncthreads();  // s_lo / s_hi are the next group's
+  }
 }
 
 // Many waves per empty-space cell: the cell's neighbourhood [c*C - 1,
@@ -358,33 +497,10 @@ __global__ void minmax_init_kernel(uint32_t* mm, int n) {
   }
 }
 
-__global__ void minmax_finish_kernel(const uint32_t* mm, const BrickJob* jobs, int n,
-                                     float* brick_range) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    const int id = jobs[i].brick_id;
-    brick_range[2 * id] = (float)mm[2 * i];
-    brick_range[2 * id + 1] = (float)mm[2 * i + 1];
-  }
-}
-
 __global__ void fill_u64_kernel(unsigned long long* p, int64_t n, unsigned long long v) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     p[i] = v;
-}
-
-// N consecutive voxels with one load; a volume row starts at any multiple of
-// the voxel size, and unaligned global loads are legal on gfx950.
-template <typename T, int N>
-struct VoxelRun {
-  typedef T vec __attribute__((ext_vector_type(N), aligned(sizeof(T))));
-};
-template <typename T, int N>
-__device__ inline void load_run(const T* p, uint32_t (&out)[N]) {
-  const auto v = *(const __attribute__((address_space(1))) typename VoxelRun<T, N>::vec*)p;
-#pragma unroll
-  for (int j = 0; j < N; ++j) out[j] = v[j];
 }
 
 // Histograms of few bins (u8 volumes, bricks): one counter per bin and LDS
@@ -805,32 +921,44 @@ hipError_t launch_downsample(const void* src, int bpv, const int64_t d[3], void*
   return hipGetLastError();
 }
 
+// LDS of slot_block_row: 16 rows of 4 (n + 1) voxels (33 KiB for the largest
+// slots of u16).
+static size_t block_row_lds(int S, int bpv) { return (size_t)16 * 4 * (slot_blocks(S) + 1) * bpv; }
+
+// Block rows per work-group: one brick's rows spread until the launch has
+// about 16 work-groups per CU.
+static int extract_rows(int64_t n_jobs, int S) {
+  const int64_t n = slot_blocks(S), rows = n * n;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(rows, rows * n_jobs / 4096));
+}
+
+int64_t extract_scratch_words(int64_t n_jobs, int S) {
+  const int64_t rows = (int64_t)slot_blocks(S) * slot_blocks(S), per = extract_rows(n_jobs, S);
+  return 2 * n_jobs * ((rows + per - 1) / per);
+}
+
 hipError_t launch_extract_bricks(const void* level, int bpv, const int64_t d[3],
                                  const BrickJob* jobs, int n_jobs, void* pool,
                                  int64_t slot_stride, int B, int apron, float* brick_range,
                                  uint32_t* scratch, hipStream_t stream) {
-  const int64_t slot_elems = slot_block_elems(B + 2 * apron);
   if (n_jobs <= 0) return hipSuccess;
-  minmax_init_kernel<<<(n_jobs + 255) / 256, 256, 0, stream>>>(scratch, n_jobs);
-  int64_t chunks = (slot_elems + 8191) / 8192;
-  if (chunks > 1024) chunks = 1024;
-  if (chunks < 1) chunks = 1;
+  const int S = B + 2 * apron, n = slot_blocks(S), per = extract_rows(n_jobs, S);
+  const int parts = (n * n + per - 1) / per;
+  const size_t lds = block_row_lds(S, bpv);
   for (int j0 = 0; j0 < n_jobs; j0 += 65535) {
     const int nj = n_jobs - j0 < 65535 ? n_jobs - j0 : 65535;
-    const dim3 grid((unsigned)chunks, (unsigned)nj, 1);
+    const dim3 grid((unsigned)parts, (unsigned)nj, 1);
+    uint32_t* part = scratch + (int64_t)2 * j0 * parts;
     if (bpv == 1)
-      extract_bricks_kernel<uint8_t><<<grid, kThreads, 0, stream>>>(
-          (const uint8_t*)level, d[0], d[1], d[2], jobs + j0, (uint8_t*)pool, slot_stride, slot_elems, B, apron,
-          scratch + 2 * j0);
+      extract_bricks_kernel<uint8_t><<<grid, kThreads, lds, stream>>>(
+          (const uint8_t*)level, d[0], d[1], d[2], jobs + j0, (uint8_t*)pool, slot_stride, B, apron, per, part);
     else
-      extract_bricks_kernel<uint16_t><<<grid, kThreads, 0, stream>>>(
-          (const uint16_t*)level, d[0], d[1], d[2], jobs + j0, (uint16_t*)pool, slot_stride,
-          slot_elems, B, apron, scratch + 2 * j0);
+      extract_bricks_kernel<uint16_t><<<grid, kThreads, lds, stream>>>(
+          (const uint16_t*)level, d[0], d[1], d[2], jobs + j0, (uint16_t*)pool, slot_stride, B, apron, per, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  minmax_finish_kernel<<<(n_jobs + 255) / 256, 256, 0, stream>>>(scratch, jobs, n_jobs,
-                                                                  brick_range);
+  brick_range_kernel<<<(unsigned)n_jobs, 64, 0, stream>>>(scratch, parts, jobs, brick_range);
   return hipGetLastError();
 }
 
@@ -859,13 +987,12 @@ hipError_t launch_extract_linear_bricks(const void* level, int bpv, const int64_
 }
 
 hipError_t launch_linear_to_slot(const void* src, void* slot, int bpv, int S, hipStream_t stream) {
-  const int64_t n = slot_block_elems(S);
-  const unsigned blocks = (unsigned)((n + kThreads - 1) / kThreads);
+  const unsigned rows = (unsigned)(slot_blocks(S) * slot_blocks(S));
+  const size_t lds = block_row_lds(S, bpv);
   if (bpv == 1)
-    linear_to_slot_kernel<uint8_t><<<blocks, kThreads, 0, stream>>>((const uint8_t*)src, (uint8_t*)slot, S, n);
+    linear_to_slot_kernel<uint8_t><<<rows, kThreads, lds, stream>>>((const uint8_t*)src, (uint8_t*)slot, S);
   else
-    linear_to_slot_kernel<uint16_t><<<blocks, kThreads, 0, stream>>>((const uint16_t*)src, (uint16_t*)slot,
-                                                                      S, n);
+    linear_to_slot_kernel<uint16_t><<<rows, kThreads, lds, stream>>>((const uint16_t*)src, (uint16_t*)slot, S);
   return hipGetLastError();
 }
 
@@ -885,6 +1012,18 @@ hipError_t launch_cell_ranges(const void* level, int bpv, const int64_t d[3], in
   const int ncx = (int)((d[0] + C - 1) / C), ncy = (int)((d[1] + C - 1) / C),
             ncz = (int)((d[2] + C - 1) / C);
   const int64_t cells = (int64_t)ncx * ncy * ncz;
+  if (C >= 4 && C <= 32) {
+    const int gx = (ncx + 64 / C - 1) / (64 / C);
+    const int64_t n = (int64_t)gx * ncy * ncz;
+    const unsigned groups = (unsigned)std::min<int64_t>(n, (int64_t)1 << 20);
+    if (bpv == 1)
+      cell_range_small_kernel<uint8_t><<<groups, kThreads, 0, stream>>>((const uint8_t*)level, d[0], d[1], d[2], C,
+                                                                        ncx, ncy, n, gx, out);
+    else
+      cell_range_small_kernel<uint16_t><<<groups, kThreads, 0, stream>>>((const uint16_t*)level, d[0], d[1], d[2], C,
+                                                                         ncx, ncy, n, gx, out);
+    return hipGetLastError();
+  }
   const unsigned fill_blocks = (unsigned)std::min<int64_t>((cells + kThreads - 1) / kThreads, 65536);
   fill_u32_kernel<<<fill_blocks, kThreads, 0, stream>>>(out, cells, 0xffffffffu);
   fill_u32_kernel<<<fill_blocks, kThreads, 0, stream>>>(tmp_hi, cells, 0u);

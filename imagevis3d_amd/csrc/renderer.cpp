@@ -516,7 +516,11 @@ int HipRenderer::brick_levels(const LevelPlan& plan) {
   DevBuf djobs;
   TVK_HIP(djobs.alloc(jobs.size() * sizeof(BrickJob)));
   TVK_HIP(hipMemcpyAsync(djobs.p, jobs.data(), djobs.bytes, hipMemcpyHostToDevice, stream_));
-  TVK_HIP(scratch_.alloc((size_t)total * 2 * sizeof(uint32_t)));
+  int64_t words = 0;
+  for (int l = 0; l < nl; ++l)
+    words = std::max(words, extract_scratch_words((int64_t)lods[l].grid[0] * lods[l].grid[1] * lods[l].grid[2],
+                                                  plan.slot_edge));
+  TVK_HIP(scratch_.alloc((size_t)words * sizeof(uint32_t)));
   const int64_t stride = (int64_t)(slot_bytes / bpv);
   for (int l = 0; l < nl; ++l) {
     const LodInfo& L = lods[l];
