@@ -24,9 +24,10 @@ bool pinned(const void* p) {
 
 }  // namespace
 
-bool HostPipe::ready(int device) {
+bool HostPipe::ready(int device, size_t bytes) {
   if (buf_[0]) return device_ == device;
   if (tried_) return false;  // no memory for the buffers: the runtime's path
+  if ((moved_ += bytes) < kWorth) return false;
   tried_ = true;
   MemMan& mm = MemMan::ForDevice(device);
   if (!mm.ReserveCPU(kSlots * kChunk)) return false;
@@ -44,6 +45,7 @@ bool HostPipe::ready(int device) {
 }
 
 void HostPipe::Release() {
+  moved_ = 0;
   if (device_ < 0) return;
   for (int i = 0; i < kSlots; ++i) {
     if (ev_[i]) {
@@ -60,7 +62,7 @@ void HostPipe::Release() {
 }
 
 hipError_t HostPipe::Upload(int device, void* dst, const void* src, size_t bytes, hipStream_t stream) {
-  if (bytes >= kLeast && !pinned(src) && ready(device)) {
+  if (bytes >= kLeast && !pinned(src) && ready(device, bytes)) {
     const size_t n = (bytes + kChunk - 1) / kChunk;
     std::atomic<int> err{hipSuccess};
     const bool done = MemMan::ForDevice(device).TryParallelFor((size_t)kSlots, kSlots, [&](size_t t) {
@@ -87,7 +89,7 @@ hipError_t HostPipe::Download(int device, const CopyPiece* pieces, size_t n, hip
     total += pieces[i].bytes;
     direct = direct || pinned(pieces[i].dst);
   }
-  if (total >= kLeast && !direct && ready(device)) {
+  if (total >= kLeast && !direct && ready(device, total)) {
     std::vector<CopyPiece> cut;
     for (size_t i = 0; i < n; ++i)
       for (size_t off = 0; off < pieces[i].bytes; off += kChunk)

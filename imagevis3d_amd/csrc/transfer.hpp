@@ -19,15 +19,19 @@ struct CopyPiece {
 };
 
 // One stream's staging buffers: kSlots pinned buffers of kChunk bytes (16
-// MiB, counted against the device's CPU budget), made at the first large
-// copy and given back with the owner.  Used by one thread at a time, like
-// the renderer it belongs to.
+// MiB, counted against the device's CPU budget), made when the owner's large
+// copies have come to kWorth bytes and given back with the owner.  Used by
+// one thread at a time, like the renderer it belongs to.
 class HostPipe {
  public:
   static constexpr size_t kChunk = 2u << 20;
   static constexpr int kSlots = 8;
   // Smaller copies take the runtime's path: waking the workers costs more.
   static constexpr size_t kLeast = 4u << 20;
+  // Making and freeing the buffers takes about 1.2 ms, which the pinned path
+  // wins back over 35 (device to host) to 85 MB: a renderer that loads 4 MiB
+  // and goes took 1.55 ms for both against 0.48 without the buffers.
+  static constexpr size_t kWorth = 64u << 20;
 
   ~HostPipe() { Release(); }
   // Queues the copy on `stream`; `src` has been read when it returns, the
@@ -39,9 +43,10 @@ class HostPipe {
   void Release();
 
  private:
-  bool ready(int device);
+  bool ready(int device, size_t bytes);
   int device_ = -1;
   bool tried_ = false;
+  size_t moved_ = 0;  // large copies made without the buffers
   void* buf_[kSlots] = {};
   hipEvent_t ev_[kSlots] = {};
 };

@@ -66,3 +66,17 @@ def test_cell_ranges_skip_only_air(brick, cell, bits):
     # slack: sample positions that round to the other side of a cell face
     assert abs(int(ea) - int(ns.sum())) <= 2e-3 * ns.sum() + 64
     r.cleanup()
+
+
+def test_copies_before_and_after_the_pinned_buffers():
+    """A renderer's first large copies go the plain way, the later ones
+    through pinned buffers in pieces: both carry every byte, odd tails
+    included."""
+    rng = np.random.default_rng(31)
+    v = rng.integers(0, 1 << 16, (257, 259, 263)).astype(np.uint16)  # 35 MB, no multiple of a piece
+    r = gpu_renderer(None, 64, 64)
+    for k in range(3):
+        print(f"case copy {k}", flush=True)
+        r.setVolume(v + np.uint16(k), 128, 2, 1)
+        assert np.array_equal(r.readLOD(0), v + np.uint16(k))
+    r.cleanup()
