@@ -28,7 +28,8 @@
 //    in the page table and marches the cell's samples with trilinear
 //    fetches from the slot, whose apron keeps every fetch brick-local.
 //    Samples are gathered BATCH at a time so a wave keeps several gathers in
-//    flight.  Rays stop at the early-termination opacity.
+//    flight; the gradient marches put four lanes on a ray, a sample each.
+//    Rays stop at the early-termination opacity.
 //
 // The sample positions, segment lengths, opacity correction and blending
 // follow the model stated in oracle/oracle.c (the FP64 oracle it is tested
@@ -1940,8 +1941,8 @@ hipError_t launch_one(const LaunchInfo& li, const JobTable* tab, hipStream_t str
   int per_cu = 0;
   // Work-group size: 8 waves when the 1D TF is staged in LDS (64 KB per
   // work-group, so two fit a CU's 160 KB); otherwise li.wg_waves (4 or 8).
-  // The variants without an LDS TF take 114-173 VGPRs (2-4 waves per SIMD;
-  // the gradient marches 114-128 at 1 sample per batch): 8-wave
+  // The variants without an LDS TF take 91-162 VGPRs (3-5 waves per SIMD;
+  // the grouped marches most, the lone quad march is held to 128): 8-wave
   // work-groups fit a CU once or twice, 4-wave ones up to four times,
   // which is faster on cache-friendly volumes and slower where more waves
   // in flight thrash the caches (the autotuner picks).
