@@ -721,7 +721,7 @@ __global__ __launch_bounds__(kThreads) void hist2d_kernel(const T* __restrict__ 
 // counters two to a 32-bit word (up to 65536 bins = 128 KiB, so one
 // work-group of 16 waves per CU), and adds its non-zero bins to the global
 // u64 histogram at its end.  A counter that reaches 0x8000 hands 0x8000 on
-// to the global bin at once; a work-group meets a barrier after at most
+// to the global bin after the run that took it there; a work-group meets a barrier after at most
 // kHistChunk counts, so a counter never passes 0x8000 + kHistChunk before
 // the hand-over that its crossing started is done.  Lanes that share the
 // first lane's bin add once for all of them: in scans most of a wave's
