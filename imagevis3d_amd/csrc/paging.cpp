@@ -97,22 +97,25 @@ int HipRenderer::SetPagedVolume(const uint64_t dims[3], uint32_t bits, uint32_t 
   TVK_HIP(pool_.page_table.alloc((size_t)total * sizeof(uint64_t)));
   TVK_HIP(pool_.brick_range.alloc((size_t)total * 2 * sizeof(float)));
   TVK_HIP(cell_range_.alloc((size_t)plan.total_cells * sizeof(uint32_t)));
-  const size_t req_words = ((size_t)total + 1) / 2;  // cleared as u64 words
+  const size_t req_words = ((size_t)total + 1) / 2;  // both are cleared as u64 words
   TVK_HIP(requests_dev_.alloc(req_words * 8));
-  TVK_HIP(touch_dev_.alloc((size_t)total * sizeof(uint32_t)));
+  TVK_HIP(touch_dev_.alloc(req_words * 8));
   pool_.n_slots = quota;
   pool_.slot_bytes = plan.slot_bytes;
   pool_bytes_req_ = pool_bytes;
   pool_.resident = 0;
   pool_.page_table_h.assign((size_t)total, 0);
   pool_.brick_slot.assign((size_t)total, -1);
-  TVK_HIP(hipMemcpy(pool_.page_table.p, pool_.page_table_h.data(), (size_t)total * 8,
-                    hipMemcpyHostToDevice));
-  TVK_HIP(hipMemcpy(pool_.brick_range.p, pool_.brick_range_h.data(), (size_t)total * 8,
-                    hipMemcpyHostToDevice));
-  TVK_HIP(hipMemcpy(cell_range_.p, cell_init_h_.data(), cell_init_h_.size() * 4,
-                    hipMemcpyHostToDevice));
-  TVK_HIP(hipMemset(touch_dev_.p, 0, touch_dev_.bytes));
+  // on the renderer's stream, as every copy of the library: a call on the
+  // null stream fails while any other thread captures a graph
+  TVK_HIP(hipMemcpyAsync(pool_.page_table.p, pool_.page_table_h.data(), (size_t)total * 8,
+                         hipMemcpyHostToDevice, stream_));
+  TVK_HIP(hipMemcpyAsync(pool_.brick_range.p, pool_.brick_range_h.data(), (size_t)total * 8,
+                         hipMemcpyHostToDevice, stream_));
+  TVK_HIP(hipMemcpyAsync(cell_range_.p, cell_init_h_.data(), cell_init_h_.size() * 4,
+                         hipMemcpyHostToDevice, stream_));
+  TVK_HIP(launch_fill_u64(touch_dev_.as<unsigned long long>(), (int64_t)req_words, 0ull, stream_));
+  TVK_HIP(hipStreamSynchronize(stream_));
   if (requests_h_count_ < (uint64_t)total) {
     if (requests_h_) (void)hipHostFree(requests_h_);
     requests_h_ = nullptr;
@@ -250,7 +253,8 @@ int HipRenderer::sync_page_table_locked() {
 
 int HipRenderer::touch_sampled() {
   std::vector<uint32_t> touch((size_t)total_bricks_);
-  TVK_HIP(hipMemcpy(touch.data(), touch_dev_.p, touch.size() * 4, hipMemcpyDeviceToHost));
+  TVK_HIP(hipMemcpyAsync(touch.data(), touch_dev_.p, touch.size() * 4, hipMemcpyDeviceToHost, stream_));
+  TVK_HIP(hipStreamSynchronize(stream_));
   std::vector<int64_t> used;
   {
     std::lock_guard<std::mutex> g(pool_mu_);

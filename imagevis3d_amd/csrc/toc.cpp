@@ -360,7 +360,7 @@ int toc_build(int device, const void* voxels, const uint64_t dims[3], uint32_t b
 
   TOC_HIP(hipSetDevice(device));
   hipStream_t stream = nullptr;
-  TOC_HIP(hipStreamCreate(&stream));
+  TOC_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   struct StreamGuard {
     hipStream_t s;
     ~StreamGuard() {

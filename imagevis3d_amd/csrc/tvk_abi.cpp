@@ -162,19 +162,28 @@ int tvk_generate_volume_gpu(int device, int kind, uint64_t seed, uint64_t nx, ui
     tvk::set_last_error("device allocation for the generator failed");
     return TVK_ERR_OOM;
   }
+  hipStream_t stream = nullptr;  // not the null stream: it fails beside another thread's graph capture
+  if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) {
+    (void)hipFree(buf);
+    tvk::set_last_error("stream creation for the generator failed");
+    return TVK_ERR_HIP;
+  }
   const int64_t d[3] = {(int64_t)nx, (int64_t)ny, (int64_t)nz};
   int rc = TVK_OK;
   for (uint64_t z0 = 0; z0 < nz && rc == TVK_OK; z0 += slab) {
     const uint64_t cnt = std::min(slab, nz - z0);
     hipError_t e = tvk::launch_generate_volume(kind, seed, d, (int)bits, (int64_t)z0, (int64_t)cnt,
-                                               buf, nullptr);
+                                               buf, stream);
     if (e == hipSuccess)
-      e = hipMemcpy((uint8_t*)out + z0 * plane, buf, cnt * plane, hipMemcpyDeviceToHost);
+      e = hipMemcpyAsync((uint8_t*)out + z0 * plane, buf, cnt * plane, hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) {
       tvk::set_last_error(std::string("device volume generator: ") + hipGetErrorString(e));
       rc = TVK_ERR_HIP;
     }
   }
+  (void)hipStreamSynchronize(stream);
+  (void)hipStreamDestroy(stream);
   (void)hipFree(buf);
   return rc;
 }
@@ -919,8 +928,13 @@ int tvk_lod_mlp_create(int device, const uint16_t* w, const float* b, tvk_lod_ml
   tvk::lod_mlp_pack(w, packed.data());
   if (e == hipSuccess) e = m->w.alloc(packed.size() * 2);
   if (e == hipSuccess) e = m->b.alloc(kMlpBiases * 4);
-  if (e == hipSuccess) e = hipMemcpy(m->w.p, packed.data(), packed.size() * 2, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(m->b.p, b, kMlpBiases * 4, hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(m->w.p, packed.data(), packed.size() * 2, hipMemcpyHostToDevice, m->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(m->b.p, b, kMlpBiases * 4, hipMemcpyHostToDevice, m->stream);
+  if (m->stream) {  // also after an error: the copies read `packed` and `b`
+    const hipError_t done = hipStreamSynchronize(m->stream);
+    if (e == hipSuccess) e = done;
+  }
   if (e != hipSuccess) {
     tvk::set_last_error(std::string("lod mlp setup: ") + hipGetErrorString(e));
     tvk_lod_mlp_destroy(m);
