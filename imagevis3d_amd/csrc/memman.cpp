@@ -1,10 +1,12 @@
 // memman.cpp -- the device-wide memory manager (see memman.hpp).
 #include "memman.hpp"
 
+#include <stdint.h>
 #include <string.h>
 #include <unistd.h>
 
 #include <algorithm>
+#include <exception>
 
 namespace tvk {
 
@@ -487,16 +489,52 @@ void MemMan::worker() {
 }
 
 void MemMan::ParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn) {
-  threads = std::max(1, std::min(threads, kMaxWorkers + 1));
-  if (threads == 1 || n <= 1) {
+  if (threads <= 1 || n <= 1) {
     for (size_t i = 0; i < n; ++i) fn(i);
     return;
   }
+  ++par_waiting_;
   std::lock_guard<std::mutex> pg(par_mu_);
-  par_busy_ = true;
+  --par_waiting_;
+  run_parallel(n, threads, fn);
+}
+
+bool MemMan::TryParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn) {
+  if (threads <= 1 || n <= 1) {
+    for (size_t i = 0; i < n; ++i) fn(i);
+    return true;
+  }
+  // par_busy_ is always seen by a call from inside fn, whose own thread may
+  // hold par_mu_ and must not try it again
+  if (par_busy_ || par_waiting_ > 0) return false;
+  std::unique_lock<std::mutex> pg(par_mu_, std::try_to_lock);
+  if (!pg.owns_lock()) return false;
+  run_parallel(n, threads, fn);
+  return true;
+}
+
+void MemMan::run_parallel(size_t n, int threads, const std::function<void(size_t)>& fn) {
+  threads = std::min(threads, kMaxWorkers + 1);
+  // also when fn throws on this thread: no index is handed out any more, no
+  // worker runs fn, and the workers are free again
+  struct Job {
+    MemMan& m;
+    explicit Job(MemMan& mm) : m(mm) { m.par_busy_ = true; }
+    ~Job() {
+      std::unique_lock<std::mutex> lk(m.wmu_);
+      m.job_next_.store(SIZE_MAX);  // past the end of any job
+      m.wdone_.wait(lk, [&] { return m.job_active_ == 0; });
+      m.job_ = nullptr;
+      m.par_busy_ = false;
+    }
+  } job(*this);
   {
     std::lock_guard<std::mutex> lk(wmu_);
-    while ((int)workers_.size() < threads - 1) workers_.emplace_back([this] { worker(); });
+    try {
+      while ((int)workers_.size() < threads - 1) workers_.emplace_back([this] { worker(); });
+    } catch (const std::exception&) {
+      // no more threads: the ones there are, or this one alone, do the work
+    }
     ++job_gen_;
     job_ = &fn;
     job_n_ = n;
@@ -505,17 +543,7 @@ void MemMan::ParallelFor(size_t n, int threads, const std::function<void(size_t)
   wcv_.notify_all();
   const uint64_t tag = job_gen_ & ((1ull << (64 - kGenShift)) - 1);
   for (size_t i; take_index(tag, n, &i);) fn(i);
-  // every index has been taken; wait for the workers still running one
-  std::unique_lock<std::mutex> lk(wmu_);
-  wdone_.wait(lk, [&] { return job_active_ == 0; });
-  job_ = nullptr;
-  par_busy_ = false;
-}
-
-bool MemMan::TryParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn) {
-  if (par_busy_) return false;  // always seen by a call from inside fn
-  ParallelFor(n, threads, fn);
-  return true;
+  // every index has been taken; ~Job waits for the workers still running one
 }
 
 }  // namespace tvk

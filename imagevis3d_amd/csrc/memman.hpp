@@ -110,9 +110,11 @@ class MemMan {
   // Runs fn(0..n) on up to `threads` workers (the caller works too) and
   // returns when all are done.
   void ParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn);
-  // The same, unless the workers are busy: returns false and runs nothing.
-  // For work that may itself run inside fn (a brick source that reads
-  // another renderer's frame), where waiting for the workers would never end.
+  // The same, unless the workers are busy or someone waits for them: returns
+  // false at once and runs nothing.  For work that can be done without them
+  // and may itself run inside fn (a brick source that reads another
+  // renderer's frame), or hold what fn waits for, where waiting for the
+  // workers would never end.
   bool TryParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn);
 
  private:
@@ -171,6 +173,7 @@ class MemMan {
   // worker pool
   void worker();
   bool take_index(uint64_t tag, size_t n, size_t* i);
+  void run_parallel(size_t n, int threads, const std::function<void(size_t)>& fn);  // par_mu_ held
   std::vector<std::thread> workers_;
   std::mutex wmu_;
   std::condition_variable wcv_, wdone_;
@@ -183,6 +186,7 @@ class MemMan {
   bool stop_ = false;
   std::mutex par_mu_;  // one ParallelFor at a time
   std::atomic<bool> par_busy_{false};  // one is running
+  std::atomic<int> par_waiting_{0};    // ParallelFor calls that wait for par_mu_
 };
 
 }  // namespace tvk
