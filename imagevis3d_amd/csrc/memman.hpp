@@ -116,6 +116,8 @@ class MemMan {
   // renderer's frame), or hold what fn waits for, where waiting for the
   // workers would never end.
   bool TryParallelFor(size_t n, int threads, const std::function<void(size_t)>& fn);
+  // Someone waits in ParallelFor: a long TryParallelFor job should end early.
+  bool WorkersWanted() const { return par_waiting_ > 0; }
 
  private:
   explicit MemMan(int device);

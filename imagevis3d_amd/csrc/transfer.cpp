@@ -5,7 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
-#include <vector>
+#include <functional>
 
 #include "memman.hpp"
 
@@ -20,6 +20,44 @@ bool pinned(const void* p) {
     return false;
   }
   return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged;
+}
+
+// Runs piece(c, slot) for pieces [0, n) on the workers: slot t has the pieces
+// t, t + kSlots, .. from next[t] on, one after the other, and stops early
+// when someone else needs the workers.  False, and nothing done, when they
+// are busy.
+template <typename F>
+bool pooled(int device, size_t n, size_t (&next)[HostPipe::kSlots], const F& piece, hipError_t* err) {
+  MemMan& mm = MemMan::ForDevice(device);
+  std::atomic<int> first{hipSuccess};
+  const bool ran = mm.TryParallelFor((size_t)HostPipe::kSlots, HostPipe::kSlots, [&](size_t t) {
+    hipError_t e = hipSetDevice(device);
+    for (; next[t] < n && e == hipSuccess && first == hipSuccess && !mm.WorkersWanted(); next[t] += HostPipe::kSlots)
+      e = piece(next[t], t);
+    if (e != hipSuccess) first = (int)e;
+  });
+  if (ran) *err = (hipError_t)first.load();
+  return ran;
+}
+
+// All of [0, n): by `piece` on the workers, or, a few at a time while they
+// are busy, by `plain` on this thread.
+template <typename F, typename G>
+hipError_t all_pieces(int device, size_t n, const F& piece, const G& plain) {
+  size_t next[HostPipe::kSlots];
+  for (size_t t = 0; t < HostPipe::kSlots; ++t) next[t] = t;
+  hipError_t e = hipSuccess;
+  for (bool left = true; left && e == hipSuccess;) {
+    if (!pooled(device, n, next, piece, &e))
+      for (size_t t = 0; t < HostPipe::kSlots && e == hipSuccess; ++t)
+        if (next[t] < n) {
+          e = plain(next[t], t);
+          next[t] += HostPipe::kSlots;
+        }
+    left = false;
+    for (size_t k : next) left = left || k < n;
+  }
+  return e;
 }
 
 }  // namespace
@@ -62,24 +100,24 @@ void HostPipe::Release() {
 }
 
 hipError_t HostPipe::Upload(int device, void* dst, const void* src, size_t bytes, hipStream_t stream) {
-  if (bytes >= kLeast && !pinned(src) && ready(device, bytes)) {
-    const size_t n = (bytes + kChunk - 1) / kChunk;
-    std::atomic<int> err{hipSuccess};
-    const bool done = MemMan::ForDevice(device).TryParallelFor((size_t)kSlots, kSlots, [&](size_t t) {
-      hipError_t e = hipSetDevice(device);
-      for (size_t c = t; c < n && e == hipSuccess && err == hipSuccess; c += kSlots) {
-        const size_t off = c * kChunk, len = std::min(kChunk, bytes - off);
-        e = hipEventSynchronize(ev_[t]);  // the buffer's last copy (an event never recorded is done)
-        if (e != hipSuccess) break;
-        memcpy(buf_[t], (const char*)src + off, len);
-        e = hipMemcpyAsync((char*)dst + off, buf_[t], len, hipMemcpyHostToDevice, stream);
-        if (e == hipSuccess) e = hipEventRecord(ev_[t], stream);
-      }
-      if (e != hipSuccess) err = (int)e;
-    });
-    if (done) return (hipError_t)err.load();
-  }
-  return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
+  if (bytes < kLeast || pinned(src) || !ready(device, bytes))
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
+  hipError_t e = hipStreamSynchronize(stream);
+  if (e != hipSuccess) return e;
+  auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
+  auto piece = [&](size_t c, size_t t) {
+    hipError_t q = hipEventSynchronize(ev_[t]);  // the buffer's last copy (an event never recorded is done)
+    if (q != hipSuccess) return q;
+    memcpy(buf_[t], (const char*)src + c * kChunk, len(c));
+    q = hipMemcpyAsync((char*)dst + c * kChunk, buf_[t], len(c), hipMemcpyHostToDevice, stream);
+    return q == hipSuccess ? hipEventRecord(ev_[t], stream) : q;
+  };
+  auto plain = [&](size_t c, size_t) {
+    return hipMemcpyAsync((char*)dst + c * kChunk, (const char*)src + c * kChunk, len(c), hipMemcpyHostToDevice, stream);
+  };
+  e = all_pieces(device, (bytes + kChunk - 1) / kChunk, piece, plain);
+  if (e != hipSuccess) (void)hipStreamSynchronize(stream);  // nothing reads the buffers any more
+  return e;
 }
 
 hipError_t HostPipe::Download(int device, const CopyPiece* pieces, size_t n, hipStream_t stream) {
@@ -89,38 +127,58 @@ hipError_t HostPipe::Download(int device, const CopyPiece* pieces, size_t n, hip
     total += pieces[i].bytes;
     direct = direct || pinned(pieces[i].dst);
   }
-  if (total >= kLeast && !direct && ready(device, total)) {
-    std::vector<CopyPiece> cut;
+  if (total < kLeast || direct || !ready(device, total)) {
     for (size_t i = 0; i < n; ++i)
-      for (size_t off = 0; off < pieces[i].bytes; off += kChunk)
-        cut.push_back(CopyPiece{(char*)pieces[i].dst + off, (const char*)pieces[i].src + off,
-                                std::min(kChunk, pieces[i].bytes - off)});
-    std::atomic<int> err{hipSuccess};
-    const bool done = MemMan::ForDevice(device).TryParallelFor((size_t)kSlots, kSlots, [&](size_t t) {
-      hipError_t e = hipSetDevice(device);
-      for (size_t c = t; c < cut.size() && e == hipSuccess && err == hipSuccess; c += kSlots) {
-        e = hipMemcpyAsync(buf_[t], cut[c].src, cut[c].bytes, hipMemcpyDeviceToHost, stream);
-        if (e == hipSuccess) e = hipEventRecord(ev_[t], stream);
-        if (e == hipSuccess) e = hipEventSynchronize(ev_[t]);
-        if (e == hipSuccess) memcpy(cut[c].dst, buf_[t], cut[c].bytes);
-      }
-      if (e != hipSuccess) err = (int)e;
-    });
-    if (done) return (hipError_t)err.load();
+      if (hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, stream))
+        return e;
+    return hipStreamSynchronize(stream);
   }
-  for (size_t i = 0; i < n; ++i)
-    if (hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, stream))
-      return e;
-  return hipStreamSynchronize(stream);
+  size_t m = 0;  // pieces of at most kChunk bytes, each of one image
+  for (size_t i = 0; i < n; ++i) m += (pieces[i].bytes + kChunk - 1) / kChunk;
+  auto cut = [&](size_t c) {
+    size_t i = 0;
+    for (size_t k; c >= (k = (pieces[i].bytes + kChunk - 1) / kChunk); c -= k) ++i;
+    const size_t off = c * kChunk;
+    return CopyPiece{(char*)pieces[i].dst + off, (const char*)pieces[i].src + off, std::min(kChunk, pieces[i].bytes - off)};
+  };
+  auto fetch = [&](size_t c, size_t t) {
+    const CopyPiece p = cut(c);
+    const hipError_t q = hipMemcpyAsync(buf_[t], p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+    return q == hipSuccess ? hipEventRecord(ev_[t], stream) : q;
+  };
+  auto drain = [&](size_t c, size_t t) {
+    const CopyPiece p = cut(c);
+    const hipError_t q = hipEventSynchronize(ev_[t]);
+    if (q == hipSuccess) memcpy(p.dst, buf_[t], p.bytes);
+    return q;
+  };
+  // each slot's first piece follows the stream's work at once; the workers
+  // are taken when that work and the first piece are done
+  const size_t ahead = std::min(m, (size_t)kSlots);
+  hipError_t e = hipSuccess;
+  for (size_t c = 0; c < ahead && e == hipSuccess; ++c) e = fetch(c, c);
+  if (e == hipSuccess) e = hipEventSynchronize(ev_[0]);
+  auto piece = [&](size_t c, size_t t) {
+    const hipError_t q = c < ahead ? hipSuccess : fetch(c, t);
+    return q == hipSuccess ? drain(c, t) : q;
+  };
+  auto plain = [&](size_t c, size_t t) {
+    const CopyPiece p = cut(c);
+    return c < ahead ? drain(c, t) : hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+  };
+  if (e == hipSuccess) e = all_pieces(device, m, piece, plain);
+  const hipError_t last = hipStreamSynchronize(stream);  // the copies made without the workers, or an error's
+  return e == hipSuccess ? last : e;
 }
 
 void parallel_memcpy(int device, void* dst, const void* src, size_t bytes) {
   constexpr size_t kPart = 1u << 20;
   const size_t n = (bytes + kPart - 1) / kPart;
-  if (bytes < HostPipe::kLeast || !MemMan::ForDevice(device).TryParallelFor(n, HostPipe::kSlots, [&](size_t i) {
-        const size_t off = i * kPart;
-        memcpy((char*)dst + off, (const char*)src + off, std::min(kPart, bytes - off));
-      }))
+  auto part = [&](size_t i) {
+    const size_t off = i * kPart;
+    memcpy((char*)dst + off, (const char*)src + off, std::min(kPart, bytes - off));
+  };
+  if (bytes < HostPipe::kLeast || !MemMan::ForDevice(device).TryParallelFor(n, HostPipe::kSlots, std::ref(part)))
     memcpy(dst, src, bytes);
 }
 

@@ -4,7 +4,10 @@
 // pinned buffers with one thread: 28 GB/s to the device and 17 GB/s back on
 // this machine, where pinned copies reach 57 GB/s both ways.  Here worker
 // threads move the pieces between the caller's memory and a pinned buffer
-// each while other pieces are on the link.
+// each while other pieces are on the link.  The workers serve the whole
+// device (paging needs them too): a transfer takes them once the work queued
+// before it is done and gives them up, after the pieces at hand, to anyone
+// who waits for them; while they are busy, pieces go the runtime's way.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -34,8 +37,8 @@ class HostPipe {
   static constexpr size_t kWorth = 64u << 20;
 
   ~HostPipe() { Release(); }
-  // Queues the copy on `stream`; `src` has been read when it returns, the
-  // device data is there in stream order.
+  // Queues the copy on `stream`; `src` stays as it is until the stream has
+  // passed the copy.
   hipError_t Upload(int device, void* dst, const void* src, size_t bytes, hipStream_t stream);
   // Copies device memory out after the work queued on `stream`; the data is
   // in host memory when it returns.

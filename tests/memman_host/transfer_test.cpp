@@ -1,0 +1,106 @@
+// Large host copies (imagevis3d_amd/csrc/transfer.cpp) on the host, with
+// hip_stub.cpp and transfer_stub.cpp standing in for the device: every byte
+// arrives, and the device's workers are not held while a frame renders nor for a
+// whole transfer.  Built with AddressSanitizer by
+// tests/test_transfer_host.py.  TEST INFRASTRUCTURE ONLY.
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <thread>
+#include <vector>
+
+#include "../../imagevis3d_amd/csrc/memman.hpp"
+#include "../../imagevis3d_amd/csrc/transfer.hpp"
+#include "transfer_stub.hpp"
+
+using tvk::CopyPiece;
+using tvk::HostPipe;
+using tvk::MemMan;
+
+#define CHECK(c)                                                            \
+  do {                                                                      \
+    if (!(c)) {                                                             \
+      fprintf(stderr, "%s:%d: check failed: %s\n", __FILE__, __LINE__, #c); \
+      exit(1);                                                              \
+    }                                                                       \
+  } while (0)
+
+static const size_t MiB = 1u << 20;
+
+static std::vector<unsigned char> pattern(size_t n, unsigned seed) {
+  std::vector<unsigned char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = (unsigned char)((i * 2654435761u + seed) >> 13);
+  return v;
+}
+
+int main() {
+  MemMan& mm = MemMan::ForDevice(0);
+  HostPipe pipe;
+  {  // sizes around pieces, the first ones before the buffers are there
+    for (size_t n : {5 * MiB + 1, 70 * MiB + 3, 64 * MiB, 4 * MiB, 130 * MiB - 1, 3 * MiB, (size_t)1}) {
+      const std::vector<unsigned char> src = pattern(n, (unsigned)n);
+      std::vector<unsigned char> up(n), down(n);
+      CHECK(pipe.Upload(0, up.data(), src.data(), n, nullptr) == hipSuccess && up == src);
+      const CopyPiece piece{down.data(), src.data(), n};
+      CHECK(pipe.Download(0, &piece, 1, nullptr) == hipSuccess && down == src);
+    }
+    CHECK(g_pinned == HostPipe::kSlots * HostPipe::kChunk);
+    printf("OK sizes\n");
+  }
+  {  // many images, empty ones among them
+    const std::vector<unsigned char> src = pattern(90 * MiB, 5);
+    std::vector<unsigned char> down(src.size());
+    std::vector<CopyPiece> pieces;
+    size_t at = 0;
+    for (size_t k = 0; at < src.size(); ++k) {
+      const size_t len = std::min(src.size() - at, k % 7 == 3 ? (size_t)0 : k % 5 == 1 ? 5 * MiB + k : 100 * 1000 + k);
+      pieces.push_back(CopyPiece{down.data() + at, src.data() + at, len});
+      at += len;
+    }
+    CHECK(pieces.size() > 64);
+    CHECK(pipe.Download(0, pieces.data(), pieces.size(), nullptr) == hipSuccess && down == src);
+    printf("OK pieces\n");
+  }
+  for (int up = 0; up < 2; ++up) {  // a frame is queued before the copy: the workers are free until it is done
+    const std::vector<unsigned char> src = pattern(8 * MiB, 9);
+    std::vector<unsigned char> dst(src.size());
+    int waited = 0;
+    g_on_wait = [&] {
+      ++waited;
+      CHECK(mm.TryParallelFor(2, 2, [](size_t) {}));
+    };
+    g_frame = true;
+    const CopyPiece piece{dst.data(), src.data(), src.size()};
+    CHECK((up ? pipe.Upload(0, dst.data(), src.data(), src.size(), nullptr)
+              : pipe.Download(0, &piece, 1, nullptr)) == hipSuccess);
+    CHECK(waited == 1 && !g_frame && dst == src);
+    g_on_wait = nullptr;
+    printf("OK frame\n");
+  }
+  for (int up = 0; up < 2; ++up) {  // someone who needs the workers gets them after the pieces at hand
+    const std::vector<unsigned char> src = pattern(320 * MiB, 11);
+    std::vector<unsigned char> dst(src.size());
+    g_copied = 0;
+    size_t asked = 0, got = 0;
+    std::thread pager([&] {
+      while (g_copied < 20 * MiB) std::this_thread::yield();
+      asked = g_copied;
+      mm.ParallelFor(2, 2, [&](size_t i) {
+        if (i == 0) got = g_copied;
+      });
+    });
+    const CopyPiece piece{dst.data(), src.data(), src.size()};
+    CHECK((up ? pipe.Upload(0, dst.data(), src.data(), src.size(), nullptr)
+              : pipe.Download(0, &piece, 1, nullptr)) == hipSuccess);
+    pager.join();
+    CHECK(dst == src);
+    printf("asked at %zu MiB, got the workers at %zu MiB\n", asked / MiB, got / MiB);
+    CHECK(got <= asked + 4 * HostPipe::kSlots * HostPipe::kChunk);
+    printf("OK wanted\n");
+  }
+  pipe.Release();
+  CHECK(g_pinned == 0);
+  printf("ALL OK\n");
+  return 0;
+}

@@ -1,4 +1,4 @@
-"""Worker threads of the memory manager on the host (no GPU): the sources
+"""Worker threads of the memory manager and large host copies on the host (no GPU): the sources
 are built with host stand-ins for the HIP calls they make and
 AddressSanitizer, and C++ drivers check them."""
 import os
@@ -29,3 +29,8 @@ pytestmark = pytest.mark.skipif(shutil.which("g++") is None or not os.path.isdir
 
 def test_workers(tmp_path):
     run(tmp_path, os.path.join(HERE, "workers_test.cpp"), os.path.join(CSRC, "memman.cpp"))
+
+
+def test_large_copies(tmp_path):
+    run(tmp_path, os.path.join(HERE, "transfer_test.cpp"), os.path.join(HERE, "transfer_stub.cpp"),
+        os.path.join(CSRC, "transfer.cpp"), os.path.join(CSRC, "memman.cpp"))
