@@ -30,12 +30,14 @@ template <typename F>
 bool pooled(int device, size_t n, size_t (&next)[HostPipe::kSlots], const F& piece, hipError_t* err) {
   MemMan& mm = MemMan::ForDevice(device);
   std::atomic<int> first{hipSuccess};
-  const bool ran = mm.TryParallelFor((size_t)HostPipe::kSlots, HostPipe::kSlots, [&](size_t t) {
+  auto slot = [&](size_t t) {
     hipError_t e = hipSetDevice(device);
     for (; next[t] < n && e == hipSuccess && first == hipSuccess && !mm.WorkersWanted(); next[t] += HostPipe::kSlots)
       e = piece(next[t], t);
     if (e != hipSuccess) first = (int)e;
-  });
+  };
+  // by reference: a std::function of it needs no memory
+  const bool ran = mm.TryParallelFor((size_t)HostPipe::kSlots, HostPipe::kSlots, std::ref(slot));
   if (ran) *err = (hipError_t)first.load();
   return ran;
 }

@@ -37,8 +37,8 @@ class HostPipe {
   static constexpr size_t kWorth = 64u << 20;
 
   ~HostPipe() { Release(); }
-  // Queues the copy on `stream`; `src` stays as it is until the stream has
-  // passed the copy.
+  // Neither copy throws.  Upload queues the copy on `stream`; `src` stays as
+  // it is until the stream has passed it.
   hipError_t Upload(int device, void* dst, const void* src, size_t bytes, hipStream_t stream);
   // Copies device memory out after the work queued on `stream`; the data is
   // in host memory when it returns.

@@ -1,12 +1,13 @@
 // Large host copies (imagevis3d_amd/csrc/transfer.cpp) on the host, with
 // hip_stub.cpp and transfer_stub.cpp standing in for the device: every byte
-// arrives, and the device's workers are not held while a frame renders nor for a
-// whole transfer.  Built with AddressSanitizer by
+// arrives, the device's workers are not held while a frame renders nor for a
+// whole transfer, and no call throws.  Built with AddressSanitizer by
 // tests/test_transfer_host.py.  TEST INFRASTRUCTURE ONLY.
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -25,6 +26,15 @@ using tvk::MemMan;
       exit(1);                                                              \
     }                                                                       \
   } while (0)
+
+static thread_local bool t_no_memory = false;
+void* operator new(size_t n) {
+  void* p = t_no_memory ? nullptr : malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 static const size_t MiB = 1u << 20;
 
@@ -98,6 +108,18 @@ int main() {
     printf("asked at %zu MiB, got the workers at %zu MiB\n", asked / MiB, got / MiB);
     CHECK(got <= asked + 4 * HostPipe::kSlots * HostPipe::kChunk);
     printf("OK wanted\n");
+  }
+  {  // no memory for anything: the copies are made all the same
+    const std::vector<unsigned char> src = pattern(9 * MiB, 13);
+    std::vector<unsigned char> a(src.size()), b(src.size()), c(src.size());
+    const CopyPiece piece{b.data(), src.data(), src.size()};
+    t_no_memory = true;
+    const hipError_t e1 = pipe.Upload(0, a.data(), src.data(), src.size(), nullptr);
+    const hipError_t e2 = pipe.Download(0, &piece, 1, nullptr);
+    tvk::parallel_memcpy(0, c.data(), src.data(), src.size());
+    t_no_memory = false;
+    CHECK(e1 == hipSuccess && e2 == hipSuccess && a == src && b == src && c == src);
+    printf("OK no memory\n");
   }
   pipe.Release();
   CHECK(g_pinned == 0);
