@@ -67,6 +67,7 @@ void MemMan::SetCPUBudget(uint64_t bytes) {
     std::lock_guard<std::mutex> g(mu_);
     cpu_budget_ = bytes;
   }
+  ask_back(0, true);
   std::lock_guard<std::mutex> g(cache_mu_);
   cache_trim_locked(0);
 }
@@ -117,7 +118,35 @@ void MemMan::ReleaseGPU(uint64_t bytes) {
   gpu_used_ -= std::min(gpu_used_, bytes);
 }
 
+// No lock is held while holders give back: they may wait for copies and take
+// mu_ to return their bytes.
+void MemMan::ask_back(uint64_t bytes, bool wait) {
+  if (cpu_spare_ == 0) return;
+  {
+    std::lock_guard<std::mutex> c(cache_mu_);
+    if (cpu_used_ + cache_bytes_ + bytes <= cpu_budget_) return;
+  }
+  if (auto f = give_back_.load()) f(device_, wait);
+}
+
+bool MemMan::ReserveSpareCPU(uint64_t bytes, void (*give_back)(int, bool)) {
+  std::lock_guard<std::mutex> g(mu_);
+  std::lock_guard<std::mutex> c(cache_mu_);
+  if (cpu_used_ + cache_bytes_ + bytes > cpu_budget_) return false;
+  give_back_ = give_back;
+  cpu_used_ += bytes;
+  cpu_spare_ += bytes;
+  return true;
+}
+
+void MemMan::ReleaseSpareCPU(uint64_t bytes) {
+  std::lock_guard<std::mutex> g(mu_);
+  cpu_used_ -= std::min(cpu_used_.load(), bytes);
+  cpu_spare_ -= std::min(cpu_spare_.load(), bytes);
+}
+
 bool MemMan::ReserveCPU(uint64_t bytes) {
+  ask_back(bytes, true);
   std::lock_guard<std::mutex> g(mu_);
   {
     std::lock_guard<std::mutex> c(cache_mu_);
@@ -431,6 +460,7 @@ bool MemMan::CacheGet(int client, int gid, void* dst, uint64_t bytes) {
 }
 
 void MemMan::CachePut(int client, int gid, const void* src, uint64_t bytes) {
+  ask_back(bytes, false);
   std::lock_guard<std::mutex> g(cache_mu_);
   const uint64_t key = ((uint64_t)(uint32_t)client << 32) | (uint32_t)gid;
   if (cache_.count(key)) return;

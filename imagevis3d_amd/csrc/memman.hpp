@@ -84,6 +84,13 @@ class MemMan {
   // Host memory held for bricks outside the cache (the cache evicts itself).
   bool ReserveCPU(uint64_t bytes);
   void ReleaseCPU(uint64_t bytes);
+  // Host memory its holder can do without (staging buffers): granted only
+  // from what neither the budget's other holders nor the cache use, and asked
+  // back with give_back(wait) before anything is refused or leaves the cache
+  // for want of room.  give_back returns the memory of idle holders to
+  // ReleaseSpareCPU, with `wait` also that of the others once they are idle.
+  bool ReserveSpareCPU(uint64_t bytes, void (*give_back)(int device, bool wait));
+  void ReleaseSpareCPU(uint64_t bytes);
 
   // Paged pool.  max_slots caps the client's share (0: no cap).
   int Register(PoolClient* c, uint64_t slot_bytes, uint64_t max_slots);
@@ -155,6 +162,7 @@ class MemMan {
   void evict_slot(SlotClass& C, int64_t s);
   bool protected_for(const Slot& sl, int client) const;
   void cache_trim_locked(uint64_t room);
+  void ask_back(uint64_t bytes, bool wait);  // spare memory, unless `bytes` more fit beside it
   void* slot_addr(const SlotClass& C, int64_t s) const;
 
   int device_;
@@ -162,6 +170,8 @@ class MemMan {
   uint64_t gpu_total_ = 0, gpu_budget_ = 0, gpu_used_ = 0;
   uint64_t cpu_total_ = 0;
   std::atomic<uint64_t> cpu_budget_{0}, cpu_used_{0};  // also read by the cache without mu_
+  std::atomic<uint64_t> cpu_spare_{0};                 // of cpu_used_: can be asked back
+  std::atomic<void (*)(int, bool)> give_back_{nullptr};
   uint64_t clock_ = 1;
   uint64_t evictions_ = 0, chunks_freed_ = 0;
   std::vector<SlotClass> classes_;

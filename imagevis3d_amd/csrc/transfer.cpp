@@ -6,6 +6,9 @@
 #include <algorithm>
 #include <atomic>
 #include <functional>
+#include <map>
+#include <new>
+#include <vector>
 
 #include "memman.hpp"
 
@@ -64,29 +67,79 @@ hipError_t all_pieces(int device, size_t n, const F& piece, const G& plain) {
 
 }  // namespace
 
-bool HostPipe::ready(int device, size_t bytes) {
-  if (buf_[0]) return device_ == device;
-  if (tried_) return false;  // no memory for the buffers: the runtime's path
-  if ((moved_ += bytes) < kWorth) return false;
-  tried_ = true;
-  MemMan& mm = MemMan::ForDevice(device);
-  if (!mm.ReserveCPU(kSlots * kChunk)) return false;
-  device_ = device;
-  bool ok = true;
-  for (int i = 0; i < kSlots && ok; ++i)
-    ok = hipHostMalloc(&buf_[i], kChunk, hipHostMallocDefault) == hipSuccess &&
-         hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming) == hipSuccess;
-  if (!ok) {
-    (void)hipGetLastError();
-    Release();
-    tried_ = true;
-  }
-  return ok;
+// The pipes of a device, asked to give their buffers back.  Its lock is not
+// taken by a pipe in a transfer.
+struct HostPipes {
+  std::mutex mu;
+  std::vector<HostPipe*> all;
+};
+static HostPipes& pipes_of(int device) {
+  static std::mutex m;
+  static std::map<int, HostPipes*> all;  // for the life of the process, as the memory managers
+  std::lock_guard<std::mutex> g(m);
+  auto it = all.find(device);
+  if (it == all.end()) it = all.emplace(device, new HostPipes()).first;
+  return *it->second;
 }
 
-void HostPipe::Release() {
-  moved_ = 0;
-  if (device_ < 0) return;
+// A transfer's use of the buffers.
+struct HostPipe::Loan {
+  HostPipe& p;
+  const bool ok;
+  Loan(HostPipe& pipe, int device, size_t bytes) : p(pipe), ok(pipe.begin(device, bytes)) {}
+  ~Loan() {
+    if (ok) p.end();
+  }
+};
+
+bool HostPipe::begin(int device, size_t bytes) {
+  if (device_ >= 0 && device_ != device) return false;
+  {
+    std::lock_guard<std::mutex> g(mu_);
+    if (!buf_[0]) {
+      if ((moved_ += bytes) < kWorth) return false;
+      moved_ = 0;
+    }
+  }
+  if (device_ < 0) {
+    try {
+      HostPipes& P = pipes_of(device);
+      std::lock_guard<std::mutex> g(P.mu);
+      P.all.push_back(this);
+    } catch (const std::bad_alloc&) {
+      return false;
+    }
+    device_ = device;
+  }
+  {
+    std::lock_guard<std::mutex> g(mu_);
+    busy_ = true;
+  }
+  if (buf_[0]) return true;
+  // no room or no memory for the buffers: the runtime's path
+  if (MemMan::ForDevice(device).ReserveSpareCPU(kSlots * kChunk, &HostPipe::give_back)) {
+    bool ok = true;
+    for (int i = 0; i < kSlots && ok; ++i)
+      ok = hipHostMalloc(&buf_[i], kChunk, hipHostMallocDefault) == hipSuccess &&
+           hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming) == hipSuccess;
+    if (ok) return true;
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> g(mu_);
+    drop();
+  }
+  end();
+  return false;
+}
+
+void HostPipe::end() {
+  {
+    std::lock_guard<std::mutex> g(mu_);
+    busy_ = false;
+  }
+  idle_.notify_all();
+}
+
+void HostPipe::drop() {
   for (int i = 0; i < kSlots; ++i) {
     if (ev_[i]) {
       (void)hipEventSynchronize(ev_[i]);  // its last copy may still read the buffer
@@ -96,14 +149,39 @@ void HostPipe::Release() {
     ev_[i] = nullptr;
     buf_[i] = nullptr;
   }
-  MemMan::ForDevice(device_).ReleaseCPU(kSlots * kChunk);
+  moved_ = 0;
+  MemMan::ForDevice(device_).ReleaseSpareCPU(kSlots * kChunk);
+}
+
+void HostPipe::give(bool wait) {
+  std::unique_lock<std::mutex> lk(mu_);
+  if (busy_ && !wait) return;
+  idle_.wait(lk, [&] { return !busy_; });
+  if (buf_[0]) drop();
+}
+
+void HostPipe::give_back(int device, bool wait) {
+  HostPipes& P = pipes_of(device);
+  std::lock_guard<std::mutex> g(P.mu);
+  for (HostPipe* p : P.all) p->give(wait);
+}
+
+void HostPipe::Release() {
+  if (device_ >= 0) {
+    HostPipes& P = pipes_of(device_);
+    std::lock_guard<std::mutex> g(P.mu);
+    P.all.erase(std::find(P.all.begin(), P.all.end(), this));
+  }
+  std::lock_guard<std::mutex> g(mu_);
+  if (buf_[0]) drop();
+  moved_ = 0;
   device_ = -1;
-  tried_ = false;
 }
 
 hipError_t HostPipe::Upload(int device, void* dst, const void* src, size_t bytes, hipStream_t stream) {
-  if (bytes < kLeast || pinned(src) || !ready(device, bytes))
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
+  if (bytes < kLeast || pinned(src)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
+  const Loan loan(*this, device, bytes);
+  if (!loan.ok) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
   hipError_t e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return e;
   auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
@@ -129,12 +207,15 @@ hipError_t HostPipe::Download(int device, const CopyPiece* pieces, size_t n, hip
     total += pieces[i].bytes;
     direct = direct || pinned(pieces[i].dst);
   }
-  if (total < kLeast || direct || !ready(device, total)) {
+  auto by_runtime = [&] {
     for (size_t i = 0; i < n; ++i)
       if (hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, stream))
         return e;
     return hipStreamSynchronize(stream);
-  }
+  };
+  if (total < kLeast || direct) return by_runtime();
+  const Loan loan(*this, device, total);
+  if (!loan.ok) return by_runtime();
   size_t m = 0;  // pieces of at most kChunk bytes, each of one image
   for (size_t i = 0; i < n; ++i) m += (pieces[i].bytes + kChunk - 1) / kChunk;
   auto cut = [&](size_t c) {

@@ -13,6 +13,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <condition_variable>
+#include <mutex>
+
 namespace tvk {
 
 struct CopyPiece {
@@ -22,9 +25,10 @@ struct CopyPiece {
 };
 
 // One stream's staging buffers: kSlots pinned buffers of kChunk bytes (16
-// MiB, counted against the device's CPU budget), made when the owner's large
-// copies have come to kWorth bytes and given back with the owner.  Used by
-// one thread at a time, like the renderer it belongs to.
+// MiB of the device's CPU budget that nobody else uses), made when the
+// owner's large copies have come to kWorth bytes and given back with the
+// owner, or when the budget is needed for anything else.  Used by one thread
+// at a time, like the renderer it belongs to.
 class HostPipe {
  public:
   static constexpr size_t kChunk = 2u << 20;
@@ -46,10 +50,17 @@ class HostPipe {
   void Release();
 
  private:
-  bool ready(int device, size_t bytes);
+  struct Loan;
+  bool begin(int device, size_t bytes);  // the buffers are there, and ours until end()
+  void end();
+  void give(bool wait);
+  void drop();  // frees the buffers; mu_ held
+  static void give_back(int device, bool wait);
   int device_ = -1;
-  bool tried_ = false;
-  size_t moved_ = 0;  // large copies made without the buffers
+  std::mutex mu_;  // busy_ and, while it is false, all below
+  std::condition_variable idle_;
+  bool busy_ = false;  // a transfer is using the buffers
+  size_t moved_ = 0;   // large copies made without the buffers
   void* buf_[kSlots] = {};
   hipEvent_t ev_[kSlots] = {};
 };

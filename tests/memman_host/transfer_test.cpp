@@ -1,12 +1,15 @@
 // Large host copies (imagevis3d_amd/csrc/transfer.cpp) on the host, with
 // hip_stub.cpp and transfer_stub.cpp standing in for the device: every byte
 // arrives, the device's workers are not held while a frame renders nor for a
-// whole transfer, and no call throws.  Built with AddressSanitizer by
+// whole transfer, no
+// call throws, and the buffers give way to any other use of the CPU budget.  Built with AddressSanitizer by
 // tests/test_transfer_host.py.  TEST INFRASTRUCTURE ONLY.
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
+#include <chrono>
 #include <new>
 #include <thread>
 #include <vector>
@@ -123,6 +126,78 @@ int main() {
   }
   pipe.Release();
   CHECK(g_pinned == 0);
+  // ---- the buffers use only memory that nobody else asks for
+  const size_t kBuf = HostPipe::kSlots * HostPipe::kChunk;
+  const std::vector<unsigned char> src = pattern(70 * MiB, 17);
+  std::vector<unsigned char> dst(src.size());
+  auto move = [&](HostPipe& p) {  // comes to kWorth in one copy
+    std::fill(dst.begin(), dst.end(), 0);
+    CHECK(p.Upload(0, dst.data(), src.data(), src.size(), nullptr) == hipSuccess && dst == src);
+  };
+  auto cpu_used = [&] {
+    tvk::MemManStats st;
+    mm.Stats(&st);
+    return st.cpu_used;
+  };
+  const uint64_t base = cpu_used();
+  {  // memory that is needed: every pipe gives its buffers back
+    HostPipe a, b;
+    mm.SetCPUBudget(base + 40 * MiB);
+    move(a);
+    move(b);
+    CHECK(g_pinned == 2 * kBuf && cpu_used() == base + 2 * kBuf);
+    CHECK(mm.ReserveCPU(8 * MiB) && g_pinned == 2 * kBuf);  // fits beside them
+    CHECK(mm.ReserveCPU(32 * MiB) && g_pinned == 0 && cpu_used() == base + 40 * MiB);
+    move(a);  // no room for buffers now
+    CHECK(g_pinned == 0);
+    CHECK(!mm.ReserveCPU(1));
+    mm.ReleaseCPU(40 * MiB);
+    move(a);
+    CHECK(g_pinned == kBuf);
+    mm.SetCPUBudget(base + kBuf - 1);  // a smaller budget
+    CHECK(g_pinned == 0 && cpu_used() == base);
+    printf("OK give back\n");
+  }
+  CHECK(cpu_used() == base);
+  {  // the brick cache: it grows into the buffers' memory, and they take none of its
+    HostPipe a;
+    mm.SetCPUBudget(base + 20 * MiB);
+    move(a);
+    CHECK(g_pinned == kBuf);
+    const std::vector<unsigned char> brick(MiB, 3);
+    for (int g = 0; g < 20; ++g) mm.CachePut(7, g, brick.data(), brick.size());
+    tvk::MemManStats st;
+    mm.Stats(&st);
+    CHECK(st.cache_bytes == 20 * MiB && g_pinned == 0);
+    move(a);
+    mm.Stats(&st);
+    CHECK(st.cache_bytes == 20 * MiB && g_pinned == 0);
+    mm.SetCPUBudget(base);  // empties the cache
+    mm.SetCPUBudget(1ull << 40);
+    printf("OK cache\n");
+  }
+  {  // asked in the middle of a transfer: waits for its end, not for ever
+    HostPipe a;
+    mm.SetCPUBudget(base + 30 * MiB);
+    move(a);
+    std::thread other;
+    std::atomic<int> got{-1};
+    g_on_wait = [&] {
+      other = std::thread([&] { got = mm.ReserveCPU(30 * MiB) ? 1 : 0; });
+      std::this_thread::sleep_for(std::chrono::milliseconds(100));
+      CHECK(got == -1);
+    };
+    g_frame = true;
+    const CopyPiece piece{dst.data(), src.data(), src.size()};
+    CHECK(a.Download(0, &piece, 1, nullptr) == hipSuccess && dst == src);
+    other.join();
+    g_on_wait = nullptr;
+    CHECK(got == 1 && g_pinned == 0);
+    mm.ReleaseCPU(30 * MiB);
+    mm.SetCPUBudget(1ull << 40);
+    printf("OK in a transfer\n");
+  }
+  CHECK(g_pinned == 0 && cpu_used() == base);
   printf("ALL OK\n");
   return 0;
 }
