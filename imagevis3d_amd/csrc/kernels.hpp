@@ -117,7 +117,6 @@ struct LaunchInfo {
   int lighting = 0;     // 1D TF with lighting
   int batch = 8;        // samples per gather batch (1D TF without lighting)
   int n_tf_lds = 0;     // > 0: the table's shared 1D TF goes to LDS
-  int lds_quads = 0;    // gradient launches: 16-byte units of the table's LDS tables
   int regions = 0;      // 1D TF with per-region LOD (jobs carry region codes)
   int compute_units = 0;
   int wg_waves = 4;      // waves per work-group of variants without an LDS TF (4 or 8)

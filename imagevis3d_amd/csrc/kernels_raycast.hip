@@ -1947,7 +1947,11 @@ hipError_t launch_one(const LaunchInfo& li, const JobTable* tab, hipStream_t str
   // which is faster on cache-friendly volumes and slower where more waves
   // in flight thrash the caches (the autotuner picks).
   const int kT = TF_LDS ? kThreads : 64 * (li.wg_waves == 4 ? 4 : 8);
-  if (!TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup || MODE == kModeGradLone)) lds += (size_t)li.lds_quads * sizeof(float4);
+  // Gradient launches: room for all tables whatever the launch has, so that
+  // one captured graph serves any TFs.  It costs no occupancy: at most 4 waves
+  // a SIMD by registers, 4 work-groups of 4 waves hold 134 of the CU's 160 KiB.
+  if (!TF_LDS && (MODE == kModeGrad || MODE == kModeGradGroup || MODE == kModeGradLone))
+    lds += (size_t)kLdsTableQuads * sizeof(float4);
   if (MODE == kMode1DStaged) lds += (size_t)(kT / 64) * kStageElems * sizeof(T);  // per-wave cell buffers
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kT, lds);
   if (e != hipSuccess) return e;

@@ -1660,7 +1660,7 @@ static bool same_but_tf(const RaycastParams& a, const RaycastParams& b) {
 // kGroupMax, the first of them leading); *groups = the groups formed.
 static int fill_job_table(JobTable* t, const RaycastParams* jobs, int n, const LaunchInfo& li,
                           int tile_group, int xcd_split, unsigned long long* dev_counters, bool* culled,
-                          int* groups, int* lds_quads) {
+                          int* groups) {
   t->h.n_jobs = n;
   t->h.tile_group = tile_group;
   t->h.xcd_split = xcd_split;
@@ -1679,21 +1679,19 @@ static int fill_job_table(JobTable* t, const RaycastParams* jobs, int n, const L
   // small 1D TFs go to LDS as far as they fit.  32 KiB leave room for the
   // three 4-wave work-groups per CU that the registers allow.
   t->h.n_tables = 0;
-  *lds_quads = 0;
   if (li.mode == 1 || li.lighting) {
+    int used = 0;  // 16-byte units
     for (int k = 0; k < n; ++k) {
       RaycastParams& j = t->jobs[k];
       const void* src = j.mode == 1 ? (const void*)j.tf2d_mask : (const void*)j.tf;
       const int64_t quads = j.mode == 1 ? ((int64_t)j.tf2d_w * j.tf2d_h + 127) / 128 : (int64_t)j.n_tf + 1;
       for (int m = 0; m < t->h.n_tables && j.lds_at < 0; ++m)
         if (t->h.tables[m].src == src) j.lds_at = t->h.tables[m].at;
-      if (j.lds_at >= 0 || t->h.n_tables == kLdsTables || *lds_quads + quads > kLdsTableQuads) continue;
-      j.lds_at = *lds_quads;
-      t->h.tables[t->h.n_tables++] = LdsTable{src, (int32_t)quads, *lds_quads};
-      *lds_quads += (int)quads;
+      if (j.lds_at >= 0 || t->h.n_tables == kLdsTables || used + quads > kLdsTableQuads) continue;
+      j.lds_at = used;
+      t->h.tables[t->h.n_tables++] = LdsTable{src, (int32_t)quads, used};
+      used += (int)quads;
     }
-    // whole KiB, so that launches of like TFs share a captured graph
-    *lds_quads = (*lds_quads + 63) / 64 * 64;
   }
   if (li.group) {
     for (int k = 0; k < n; ++k) {
@@ -1729,15 +1727,22 @@ static int fill_job_table(JobTable* t, const RaycastParams* jobs, int n, const L
   return total;
 }
 
+// The kernel variant that a filled table's launch runs.
+static LaunchInfo launch_variant(const LaunchInfo& li_in, int groups) {
+  LaunchInfo li = li_in;
+  li.group = groups > 0 ? 1 : 0;
+  // four lanes per ray read a small 1D TF from the launch's tables
+  if (li.lighting && li.batch != 1 && li.batch != 2) li.n_tf_lds = 0;
+  return li;
+}
+
 int launch_job_table_at(JobTable* table_h, void* dev_table, unsigned long long* dev_counters,
                         unsigned long long* counters_h, hipEvent_t ev[4], const RaycastParams* jobs, int n,
                         const LaunchInfo& li_in, int tile_group, int xcd_split, hipStream_t stream_) {
   bool culled = false;  // some job has background tiles outside its rect
-  int groups = 0, lds_quads = 0;
-  fill_job_table(table_h, jobs, n, li_in, tile_group, xcd_split, dev_counters, &culled, &groups, &lds_quads);
-  LaunchInfo li = li_in;
-  li.group = groups > 0 ? 1 : 0;
-  li.lds_quads = lds_quads;
+  int groups = 0;
+  fill_job_table(table_h, jobs, n, li_in, tile_group, xcd_split, dev_counters, &culled, &groups);
+  const LaunchInfo li = launch_variant(li_in, groups);
   const int words = kCounterBase + kJobCounters * n;
   const size_t table_bytes = offsetof(JobTable, jobs) + (size_t)n * sizeof(RaycastParams);
   TVK_HIP(hipEventRecord(ev[0], stream_));
@@ -1764,12 +1769,10 @@ int launch_job_table(LaunchSlot& sl, const RaycastParams* jobs, int n, const Lau
                                sl.ev, jobs, n, li_in, tile_group, xcd_split, stream_);
   JobTable* t = sl.table_h;
   bool culled = false;
-  int groups = 0, lds_quads = 0;
+  int groups = 0;
   fill_job_table(t, jobs, n, li_in, tile_group, xcd_split, sl.counters.as<unsigned long long>(), &culled,
-                 &groups, &lds_quads);
-  LaunchInfo li = li_in;
-  li.group = groups > 0 ? 1 : 0;
-  li.lds_quads = lds_quads;
+                 &groups);
+  const LaunchInfo li = launch_variant(li_in, groups);
   TVK_HIP(hipEventRecord(sl.ev[0], stream_));
   // Graph replay: the graph copies the whole table and all counters, so one
   // capture serves any job count; it is re-captured when the kernel
@@ -1778,7 +1781,7 @@ int launch_job_table(LaunchSlot& sl, const RaycastParams* jobs, int n, const Lau
                        (uint64_t)li.lighting << 6 | (uint64_t)li.batch << 7 | (uint64_t)li.regions << 11 |
                        (uint64_t)li.n_tf_lds << 12 |
                        (uint64_t)(li.wg_waves == 4 ? 1 : 0) << 40 | (uint64_t)li.stage << 41 |
-                       (uint64_t)li.group << 42 | (uint64_t)(li.lds_quads / 64) << 43;
+                       (uint64_t)li.group << 42;
   if (!sl.exec || sl.graph_key != key) {
     if (sl.exec) (void)hipGraphExecDestroy(sl.exec);
     if (sl.graph) (void)hipGraphDestroy(sl.graph);

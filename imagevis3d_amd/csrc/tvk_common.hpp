@@ -213,7 +213,7 @@ struct LdsTable {
   int32_t at;
 };
 constexpr int kLdsTables = 8;
-constexpr int kLdsTableQuads = 2048;  // 32 KiB for all of a launch's tables
+constexpr int kLdsTableQuads = 2048;  // 32 KiB for all of a launch's tables, in every gradient launch
 
 struct JobTableHeader {
   int32_t n_jobs;
