@@ -85,6 +85,11 @@ hipError_t launch_region_detail(const void* const* levels, const int64_t (*dims)
 hipError_t launch_fill_u64(unsigned long long* p, int64_t n, unsigned long long v,
                            hipStream_t stream);
 
+// Bytes of a 2D TF's mask (RaycastParams::tf2d_mask), whole 16-byte units.
+inline size_t tf2d_mask_bytes(size_t w, size_t h) { return (w * h + 127) / 128 * 16; }
+// The mask of a w x h 2D TF (float4 texels) in device memory.
+hipError_t launch_tf2d_mask(const float* tf2d, int w, int h, uint32_t* mask, hipStream_t stream);
+
 // Codes (u8: bit 0 empty, above it the block level) of all levels' cells for
 // one TF (mode 0/1: TF prefix counts over n_tf entries or columns; mode 2:
 // iso value).  lods_dev: lods[0..n_lod) on the device; per_brick: cells

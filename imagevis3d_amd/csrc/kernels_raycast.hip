@@ -1519,6 +1519,24 @@ __global__ __launch_bounds__(256) void cell_code_kernel(const LodInfo* __restric
   }
 }
 
+// The mask of a 2D TF: bit j w + i set where some texel of (i, j) .. (i + 1,
+// j + 1), clamped to the raster, has alpha > 0; a wave writes the two words
+// of its 64 bits.  Made on the host it took a change of a 256 x 256 TF from
+// 65 to 220 us and of a 1024 x 1024 one, with its frame, from 2.7 to 4.9 ms.
+__global__ __launch_bounds__(256) void tf2d_mask_kernel(const float4* __restrict__ tf, int w, int h, int64_t bits,
+                                                        uint32_t* __restrict__ mask) {
+  const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  bool any = false;
+  if (b < (int64_t)w * h) {
+    const int i = (int)(b % w), j = (int)(b / w);
+    const int i1 = min(i + 1, w - 1), j1 = min(j + 1, h - 1);
+    any = tf[(int64_t)j * w + i].w > 0.f || tf[(int64_t)j * w + i1].w > 0.f || tf[(int64_t)j1 * w + i].w > 0.f ||
+          tf[(int64_t)j1 * w + i1].w > 0.f;
+  }
+  const unsigned long long word = __ballot(any);
+  if ((threadIdx.x & 31) == 0 && b < bits) mask[b >> 5] = (uint32_t)(word >> (threadIdx.x & 32));
+}
+
 // Background of every pixel outside its job's tile rect (such rays miss the
 // volume box): the bytes render_tile writes for a missed ray, and no
 // dominant region.  Every work-group strides over every job's pixels, so
@@ -2010,6 +2028,12 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
 }
 
 }  // namespace
+
+hipError_t launch_tf2d_mask(const float* tf2d, int w, int h, uint32_t* mask, hipStream_t stream) {
+  const int64_t bits = (int64_t)tf2d_mask_bytes((size_t)w, (size_t)h) * 8;
+  tf2d_mask_kernel<<<(unsigned)((bits + 255) / 256), 256, 0, stream>>>((const float4*)tf2d, w, h, bits, mask);
+  return hipGetLastError();
+}
 
 hipError_t launch_cell_codes(const LodInfo* lods_dev, const LodInfo* lods, int n_lod, int per_brick,
                              const uint32_t* cell_range, const int32_t* prefix, int n_tf, float tf_scale,

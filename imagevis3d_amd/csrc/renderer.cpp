@@ -992,17 +992,6 @@ int HipRenderer::Set2DTransSlot(uint32_t slot, const float* rgba, uint32_t w, ui
     for (size_t j = 0; j < h && !any; ++j) any = rgba[4 * (j * w + i) + 3] > 0.f;
     t.prefix2d[i + 1] = t.prefix2d[i] + any;
   }
-  // the texel cells that some texel with alpha > 0 bounds
-  t.mask2d.assign((((size_t)w * h + 127) / 128) * 4, 0u);
-  for (uint32_t j = 0; j < h; ++j)
-    for (uint32_t i = 0; i < w; ++i) {
-      if (!(rgba[4 * ((size_t)j * w + i) + 3] > 0.f)) continue;
-      for (uint32_t y = j > 0 ? j - 1 : 0; y <= j; ++y)
-        for (uint32_t x = i > 0 ? i - 1 : 0; x <= i; ++x) {
-          const size_t b = (size_t)y * w + x;
-          t.mask2d[b >> 5] |= 1u << (b & 31);
-        }
-    }
   t.dirty2d = true;
   ++t.version;
   if (slot == 0) invalidate();
@@ -1111,9 +1100,9 @@ int HipRenderer::upload_tf() {
       const size_t W = t.w2d, H = t.h2d;
       if (t.tf2d_dev.bytes < W * H * 16) TVK_HIP(t.tf2d_dev.alloc(W * H * 16));
       if (t.prefix2d_dev.bytes < (W + 1) * 4) TVK_HIP(t.prefix2d_dev.alloc((W + 1) * 4));
-      if (t.mask2d_dev.bytes < t.mask2d.size() * 4) TVK_HIP(t.mask2d_dev.alloc(t.mask2d.size() * 4));
-      TVK_HIP(hipMemcpyAsync(t.mask2d_dev.p, t.mask2d.data(), t.mask2d.size() * 4, hipMemcpyHostToDevice, stream_));
+      if (t.mask2d_dev.bytes < tf2d_mask_bytes(W, H)) TVK_HIP(t.mask2d_dev.alloc(tf2d_mask_bytes(W, H)));
       TVK_HIP(hipMemcpyAsync(t.tf2d_dev.p, t.tf2d.data(), W * H * 16, hipMemcpyHostToDevice, stream_));
+      TVK_HIP(launch_tf2d_mask(t.tf2d_dev.as<float>(), (int)W, (int)H, t.mask2d_dev.as<uint32_t>(), stream_));
       TVK_HIP(hipMemcpyAsync(t.prefix2d_dev.p, t.prefix2d.data(), (W + 1) * 4, hipMemcpyHostToDevice,
                              stream_));
       t.dirty2d = false;
@@ -2135,7 +2124,7 @@ bool HipRenderer::launch_ready_without_alloc(const tvk_view* views, uint32_t n, 
     if (t.dirty2d) {
       const size_t W = t.w2d, H = t.h2d;
       if (t.tf2d_dev.bytes < W * H * 16 || t.prefix2d_dev.bytes < (W + 1) * 4 ||
-          t.mask2d_dev.bytes < t.mask2d.size() * 4)
+          t.mask2d_dev.bytes < tf2d_mask_bytes(W, H))
         return false;
     }
   }

@@ -95,8 +95,7 @@ struct TfSet {
   float max_grad = 1.f;
   bool dirty2d = false;
   DevBuf tf2d_dev, prefix2d_dev;
-  std::vector<uint32_t> mask2d;  // a bit per texel cell: some alpha > 0 (RaycastParams::tf2d_mask)
-  DevBuf mask2d_dev;
+  DevBuf mask2d_dev;      // a bit per texel cell: some alpha > 0 (RaycastParams::tf2d_mask)
   uint64_t version = 0;   // bumped by every change of this slot
   DevBuf region_code;     // per LOD-0 region: chosen level | 0x80 when TF-empty
   DevBuf region_code0;    // the same with every region at level 0
