@@ -41,7 +41,7 @@ int HipRenderer::Autotune(const tvk_view* views, uint32_t n, uint32_t flags, tvk
     ++tried;
     return TVK_OK;
   };
-  Setting cur{(uint32_t)brick_, (uint32_t)cell_, (uint32_t)batch_, 1u << tile_shift_,
+  Setting cur{(uint32_t)brick_, (uint32_t)cell_, (uint32_t)batch(), 1u << tile_shift_,
               (uint32_t)tile_group_, (uint32_t)wg_waves_, stage_ ? 1u : 0u};
   auto apply = [&](const Setting& s, bool rebrick) -> int {
     if (rebrick) {
@@ -87,17 +87,14 @@ int HipRenderer::Autotune(const tvk_view* views, uint32_t n, uint32_t flags, tvk
   // then the launch shape again for the chosen bricks: tuning the bricks
   // under the starting launch shape can settle on bricks that are only best
   // for that shape.
-  // samples per gather batch: 2 or 4 for the 1D march, 8 too with nearest
-  // sampling (trilinear runs 8 as 4); for the gradient marches (2D TF, or 1D
-  // TF with lighting) 1 or 2 per lane, or 4 = four lanes per ray; the other
-  // modes' batch is fixed
+  // samples per gather batch: 2, 4 or 8 for the 1D march; for the gradient
+  // marches (2D TF, or 1D TF with lighting) 1 or 2 per lane, or 4 = four lanes
+  // per ray; the other modes' batch is fixed
   const int mode = job_mode();
   const bool grad = mode == 1 || (mode == 0 && lighting_);
   const std::vector<uint32_t> batches =
       grad ? std::vector<uint32_t>{1u, 2u, 4u}
-           : (mode != 0 || regions_active() ? std::vector<uint32_t>{}
-                 : interp_ == TVK_LINEAR    ? std::vector<uint32_t>{2u, 4u}
-                                            : std::vector<uint32_t>{2u, 4u, 8u});
+           : (mode == 0 && !regions_active() ? std::vector<uint32_t>{2u, 4u, 8u} : std::vector<uint32_t>{});
   auto tune_launch = [&]() -> int {
     if (int e = try_values(batches, &Setting::batch, false)) return e;
     if (int e = try_values({4u, 8u, 16u}, &Setting::tile_width, false)) return e;
@@ -204,7 +201,7 @@ int HipRenderer::Autotune(const tvk_view* views, uint32_t n, uint32_t flags, tvk
     *out = tvk_tuning{};
     out->brick_size = (uint32_t)brick_;
     out->cell = (uint32_t)cell_;
-    out->samples_per_batch = (uint32_t)batch_;
+    out->samples_per_batch = (uint32_t)batch();
     out->tile_width = 1u << tile_shift_;
     out->tile_group = (uint32_t)tile_group_;
     out->xcd_split = (uint32_t)xcd_split_;

@@ -120,7 +120,7 @@ struct LaunchInfo {
   int interp = 1;       // 0 nearest, 1 trilinear
   int mode = 0;         // 0 1D TF, 1 2D TF, 2 isosurface
   int lighting = 0;     // 1D TF with lighting
-  int batch = 8;        // samples per gather batch (1D TF without lighting)
+  int batch = 4;        // samples per gather batch (1D and gradient marches)
   int n_tf_lds = 0;     // > 0: the table's shared 1D TF goes to LDS
   int regions = 0;      // 1D TF with per-region LOD (jobs carry region codes)
   int compute_units = 0;

@@ -2011,20 +2011,21 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
   if (li.stage && LINEAR && !li.lighting)
     return lds ? launch_one<T, true, 1, true, kMode1DStaged>(li, tab, stream)
                : launch_one<T, true, 1, false, kMode1DStaged>(li, tab, stream);
-  // 1D samples per gather batch: 2 or 4; 8 for nearest sampling only, whose
-  // samples are one load.  Trilinear batches of 8 take 161 VGPRs, half the
-  // waves of 4 (117), and were slower on every volume but 64^3 (159 against
-  // 165 us): a 1080p frame of 512^3 u16 829 against 640 us, 6 views 3592
-  // against 2627.  Nearest frames of 512^3: 8 in 340-362 us, 4 in 375-386.
+  // 1D samples per gather batch: 2, 4 or 8, by default (and for 1) 4 with
+  // trilinear and 8 with nearest sampling, whose samples are one load.
+  // Trilinear batches of 8 take 161 VGPRs, half the waves of 4 (117).  They
+  // win where the rays are fewer than the waves that fit (512 x 512 of 512^3
+  // u16 456 against 530 us, of 64^3 94 against 107) and lose elsewhere
+  // (1920 x 1080 of 512^3 u16 770 against 660, of 128^3 259 against 237).
+  // Nearest frames of 512^3: 8 in 340-362 us, 4 in 375-386.
   if (li.batch == 2)
     return lds ? launch_one<T, LINEAR, 2, true, kMode1D>(li, tab, stream)
                : launch_one<T, LINEAR, 2, false, kMode1D>(li, tab, stream);
-  constexpr int kMost = LINEAR ? 4 : 8;
-  if (li.batch == 4 || LINEAR)
+  if (li.batch == 4 || (LINEAR && li.batch != 8))
     return lds ? launch_one<T, LINEAR, 4, true, kMode1D>(li, tab, stream)
                : launch_one<T, LINEAR, 4, false, kMode1D>(li, tab, stream);
-  return lds ? launch_one<T, LINEAR, kMost, true, kMode1D>(li, tab, stream)
-             : launch_one<T, LINEAR, kMost, false, kMode1D>(li, tab, stream);
+  return lds ? launch_one<T, LINEAR, 8, true, kMode1D>(li, tab, stream)
+             : launch_one<T, LINEAR, 8, false, kMode1D>(li, tab, stream);
 }
 
 }  // namespace

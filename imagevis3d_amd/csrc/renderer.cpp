@@ -1529,7 +1529,7 @@ void HipRenderer::build_params(RaycastParams* p, int lod, const CameraState& cam
   }
   p->blend_bits = blend_ == TVK_BP_8BIT ? 8 : (blend_ == TVK_BP_16BIT ? 16 : 32);
   p->interp = interp_;
-  p->batch = batch_;
+  p->batch = batch();
   p->tile_group = tile_group_;
   p->xcd_split = xcd_split_;
   p->compute_units = compute_units_;
@@ -1600,7 +1600,7 @@ LaunchInfo HipRenderer::launch_info(int n_tf_lds) const {
   li.interp = interp_;
   li.mode = job_mode();
   li.lighting = (lighting_ && li.mode == 0) ? 1 : 0;
-  li.batch = batch_;
+  li.batch = batch();
   li.n_tf_lds = ((li.mode == 0 || li.mode == 3) && n_tf_lds <= 4096) ? n_tf_lds : 0;
   li.regions = (regions_active() && li.mode == 0 && !li.lighting) ? 1 : 0;
   li.compute_units = compute_units_;

@@ -500,7 +500,8 @@ class HipRenderer : public PoolClient {
   bool clip_on_ = false;
   int blend_ = TVK_BP_32BIT;
   bool skip_ = true;
-  int batch_ = 8;
+  int batch_ = 0;  // as set, 0: the default
+  int batch() const { return batch_ ? batch_ : interp_ == TVK_LINEAR ? 4 : 8; }
   int tile_group_ = 4;
   int xcd_split_ = 0;
   int wg_waves_ = 4;

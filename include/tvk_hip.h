@@ -424,12 +424,13 @@ int tvk_set_perf_measures(tvk_renderer* r, uint32_t min_framerate, int low_res_i
 int tvk_read_framebuffer(tvk_renderer* r, uint8_t* rgba, uint64_t rgba_bytes);
 
 /* Kernel launch tuning (no counterpart in the reference; chosen by the
- * autotuner): samples gathered per march step (1, 2, 4 or 8; default 8:
- * the 1D march takes 2 or 4, and 8 (or 1) as 4 with trilinear and 8 with
- * nearest sampling; the gradient marches of the 2D TF
- * and of lighting take 1 or 2 samples per lane, and any other value
- * gathers 4 consecutive samples of a ray on 4 lanes (the default);
- * the other modes take 4);
+ * autotuner): samples gathered per march step (1, 2, 4 or 8; until
+ * the first call 4 with trilinear and 8 with nearest sampling):
+ * the 1D march takes 2, 4 or 8, and 1 as that default (trilinear batches of
+ * 8 are faster on small images, slower on large ones); the gradient marches
+ * of the 2D TF and of lighting take 1 or 2 samples per lane, and any other
+ * value gathers 4 consecutive samples of a ray on 4 lanes;
+ * the other modes take 4;
  * how 8x8 ray tiles are dealt to the 8 XCDs: xcd_split 0 deals runs of
  * tile_group (1..4096) consecutive tiles round-robin, xcd_split rx in
  * {1, 2, 4, 8} gives each XCD one region of an rx x (8/rx) split of the
