@@ -2,6 +2,7 @@
 #include "server.hpp"
 
 #include <string.h>
+#include <sys/prctl.h>
 
 #include <algorithm>
 #include <chrono>
@@ -471,15 +472,22 @@ bool RenderServer::launch_locked(Lane& L) {
 
 void RenderServer::loop() {
   (void)hipSetDevice(device_);
+  // this thread's waits are tens of microseconds: let them end within one,
+  // not up to the default 50 later
+  (void)prctl(PR_SET_TIMERSLACK, 1000UL, 0UL, 0UL, 0UL);
   std::unique_lock<std::mutex> lk(mu_);
   while (true) {
     bool progress = retire_locked();
     bool busy = false;
+    double hold_ms = 0.0;  // the oldest request waits this long for company
     for (const Lane& L : lanes_) busy |= L.busy;
     for (Lane& L : lanes_) {
       if (L.busy || pending_.empty() || stop_) continue;
-      // beside launches in flight a young request waits for company
-      if (busy && (int)pending_.size() < kMaxJobs && now_ms() - reqs_[pending_.front()].t_submit < kCompanyMs) break;
+      if (busy && (int)pending_.size() < kMaxJobs) {
+        hold_ms = std::min(reqs_[pending_.front()].t_submit + kCompanyMs,
+                           reqs_[pending_.back()].t_submit + kCompanyGapMs) - now_ms();
+        if (hold_ms > 0.0) break;
+      }
       progress |= launch_locked(L);
       busy |= L.busy;
     }
@@ -491,7 +499,7 @@ void RenderServer::loop() {
       cv_work_.wait_for(lk, std::chrono::microseconds(500));
     } else if (busy) {
       // lanes in flight: poll their events at a short interval
-      cv_work_.wait_for(lk, std::chrono::microseconds(50));
+      cv_work_.wait_for(lk, std::chrono::duration<double, std::milli>(hold_ms > 0.0 ? std::min(hold_ms, 0.05) : 0.05));
     } else if (!pending_.empty() && !stop_) {
       // no lane in flight and nothing launched: the output memory is held
       // by finished requests not collected yet.  The wait gives mu_ up, so

@@ -252,3 +252,23 @@ def test_serving_mix_at_full_size_same_alone_and_in_the_mix():
     srv.close()
     for r in rs:
         r.cleanup()
+
+
+def test_a_request_nobody_follows_does_not_wait_for_company():
+    """One client with two requests in flight: a request waits for company
+    only while others keep coming."""
+    print("case serving: two requests in flight, queueing times", flush=True)
+    vols = make_volumes()[:1]
+    srv = RenderServer(arena_bytes=64 << 20, lanes=4)
+    vid = srv.addVolume(vols[0][0])
+    view = dict(view_pos=(0.3, 0.4, 1.8), view_dir=(-0.3, -0.4, -1.8), fov=45.0, width=512,
+                height=512, tf_slot=0)
+    queued, tickets = [], [srv.submit(vid, view)]
+    for _ in range(60):
+        tickets.append(srv.submit(vid, view))
+        queued.append(srv.wait(tickets.pop(0))[1].queue_ms)
+    srv.wait(tickets.pop(0))
+    print(f"median {sorted(queued)[30]:.4f} ms", flush=True)
+    assert sorted(queued)[30] < 0.09  # a wait for company lasts 0.1 ms
+    srv.close()
+    vols[0][0].cleanup()
