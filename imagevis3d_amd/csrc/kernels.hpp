@@ -42,6 +42,9 @@ hipError_t launch_slot_to_linear(const void* slot, void* dst, int bpv, int S, hi
 
 // Empty-space cell ranges of one flat level: out[(cz*ncy + cy)*ncx + cx] =
 // min | max << 16 over voxels [c*C - 1, (c+1)*C] (clamped to the level).
+// tmp_hi: as many words for the maxima while they are folded in, where
+// cell_ranges_fold(C).
+inline bool cell_ranges_fold(int C) { return C < 4 || C > 32; }
 hipError_t launch_cell_ranges(const void* level, int bpv, const int64_t dims[3], int C,
                               uint32_t* out, uint32_t* tmp_hi, hipStream_t stream);
 

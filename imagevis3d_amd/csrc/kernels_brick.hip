@@ -1023,7 +1023,7 @@ hipError_t launch_cell_ranges(const void* level, int bpv, const int64_t d[3], in
   const int ncx = (int)((d[0] + C - 1) / C), ncy = (int)((d[1] + C - 1) / C),
             ncz = (int)((d[2] + C - 1) / C);
   const int64_t cells = (int64_t)ncx * ncy * ncz;
-  if (C >= 4 && C <= 32) {
+  if (!cell_ranges_fold(C)) {
     const int gx = (ncx + 64 / C - 1) / (64 / C);
     const int64_t n = (int64_t)gx * ncy * ncz;
     const unsigned groups = (unsigned)std::min<int64_t>(n, (int64_t)1 << 20);

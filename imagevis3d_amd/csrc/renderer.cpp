@@ -531,12 +531,12 @@ int HipRenderer::brick_levels(const LevelPlan& plan) {
                                   pool_.brick_range.as<float>(), scratch_.as<uint32_t>(), stream_));
   }
   TVK_HIP(cell_range_.alloc((size_t)total_cells * sizeof(uint32_t)));
-  DevBuf cell_hi;  // the maxima while the kernel folds them in
-  TVK_HIP(cell_hi.alloc((size_t)total_cells * sizeof(uint32_t)));
+  DevBuf cell_hi;  // the maxima of large cells while they are folded in
+  if (cell_ranges_fold(cell)) TVK_HIP(cell_hi.alloc((size_t)total_cells * sizeof(uint32_t)));
   for (int l = 0; l < nl; ++l) {
     const int64_t d[3] = {lods[l].dims[0], lods[l].dims[1], lods[l].dims[2]};
     TVK_HIP(launch_cell_ranges(levels_[l].p, bpv, d, cell, cell_range_.as<uint32_t>() + lods[l].cell_base,
-                               cell_hi.as<uint32_t>() + lods[l].cell_base, stream_));
+                               cell_hi.p ? cell_hi.as<uint32_t>() + lods[l].cell_base : nullptr, stream_));
   }
   pool_.page_table_h.resize(total);
   for (int i = 0; i < total; ++i)
