@@ -504,9 +504,9 @@ __global__ void fill_u64_kernel(unsigned long long* p, int64_t n, unsigned long 
 }
 
 // Histograms of few bins (u8 volumes, bricks): one counter per bin and LDS
-// bank column, so that a wave's 64 increments never meet on an address --
-// in scans most voxels share a bin, and 64 atomics on one word are served
-// one by one (the 16-bin brick histograms of 512^3 u16: 4.34 ms with a shared
+// bank column, so that at most two of a wave's 64 increments meet on an
+// address -- in scans most voxels share a bin, and 64 atomics on one word are
+// served one by one (the 16-bin brick histograms of 512^3 u16: 4.34 ms with a shared
 // counter per bin and one work-group per brick, below 0.1 ms now).
 constexpr int kHistCols = 32;
 
@@ -721,8 +721,8 @@ __global__ __launch_bounds__(kThreads) void hist2d_kernel(const T* __restrict__ 
 // counters two to a 32-bit word (up to 65536 bins = 128 KiB, so one
 // work-group of 16 waves per CU), and adds its non-zero bins to the global
 // u64 histogram at its end.  A counter that reaches 0x8000 hands 0x8000 on
-// to the global bin after the run that took it there; a work-group meets a barrier after at most
-// kHistChunk counts, so a counter never passes 0x8000 + kHistChunk before
+// to the global bin after the run that took it there; a work-group meets a
+// barrier after at most kHistChunk counts, so a counter never passes 0x8000 + kHistChunk before
 // the hand-over that its crossing started is done.  Lanes that share the
 // first lane's bin add once for all of them: in scans most of a wave's
 // voxels are the same.

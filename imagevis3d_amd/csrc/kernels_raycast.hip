@@ -949,7 +949,8 @@ __device__ inline void render_tile(const RaycastParams& P, const float4* __restr
     // the hit inside a nested march, in each of a batch's four samples and
     // twice for ClearView, the kernel was 15,000 instructions at 140
     // registers, now 5,800 at 120: a 1080p frame of a 512^3 u16 scan 239 ->
-    // 143 us, bound by the walk to the surface and the tiles' tickets.
+    // 143 us (frames of three renderers in turn; one alone 260), of which 39%
+    // of the CU cycles see no wave: the CUs wait for the last tiles.
     if (MODE == kModeIso && cv_stage > 0) {
       float c[4];
       const float nv = iso_shade<T, LINEAR>(P, lv, o, d, Lh, hit_k, n, t0, step, lastlen, hit_v, P.iso_value,
@@ -1651,7 +1652,7 @@ constexpr int kQuadSubs = 4;   // quad waves per ray tile
 // would spill), and there the four waves of a work-group take the quarters
 // of one tile together, a barrier per tile: a quarter of the tickets, and
 // neighbouring rays share a CU's cache.  Lit 720p frame 225 -> 198 us by GM,
-// 167 by shared tiles, 152 by registers; 24 served requests 10.4 -> 9.8 ms.
+// 167 by shared tiles, 152 by registers; 24 served requests 10.4 -> 9.2 ms.
 // Groups keep a ticket per quarter: with shared tiles the 16 views of 1 GiB
 // took 22.4 ms against 21.8.
 template <typename T, bool LINEAR, int GM>
@@ -1959,8 +1960,8 @@ hipError_t launch_one(const LaunchInfo& li, const JobTable* tab, hipStream_t str
   int per_cu = 0;
   // Work-group size: 8 waves when the 1D TF is staged in LDS (64 KB per
   // work-group, so two fit a CU's 160 KB); otherwise li.wg_waves (4 or 8).
-  // The variants without an LDS TF take 91-162 VGPRs (3-5 waves per SIMD;
-  // the grouped marches most, the lone quad march is held to 128): 8-wave
+  // The variants without an LDS TF take 74-181 VGPRs (2-6 waves per SIMD;
+  // the gradient marches 124-181, the lone trilinear one held to 128): 8-wave
   // work-groups fit a CU once or twice, 4-wave ones up to four times,
   // which is faster on cache-friendly volumes and slower where more waves
   // in flight thrash the caches (the autotuner picks).
@@ -1999,8 +2000,8 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
     return li.n_tf_lds > 0 ? launch_one<T, LINEAR, 4, true, kModeMIP>(li, tab, stream)
                            : launch_one<T, LINEAR, 4, false, kModeMIP>(li, tab, stream);
   // the gradient marches: li.batch 1 or 2 samples per gather batch, each
-  // lane its own ray; otherwise four lanes per ray, a sample each (the
-  // TF-group march, which takes lone views as groups of one)
+  // lane its own ray; otherwise four lanes per ray, a sample each, with a
+  // march of its own for launches without groups
   if (li.mode == 1 || li.lighting) {
     if (li.batch == 1) return launch_grad<T, LINEAR, 1>(li, tab, stream);
     if (li.batch == 2) return launch_grad<T, LINEAR, 2>(li, tab, stream);
@@ -2013,7 +2014,7 @@ hipError_t launch_typed(const LaunchInfo& li, const JobTable* tab, hipStream_t s
                : launch_one<T, true, 1, false, kMode1DStaged>(li, tab, stream);
   // 1D samples per gather batch: 2, 4 or 8, by default (and for 1) 4 with
   // trilinear and 8 with nearest sampling, whose samples are one load.
-  // Trilinear batches of 8 take 161 VGPRs, half the waves of 4 (117).  They
+  // Trilinear batches of 8 take 174 VGPRs, half the waves of 4 (113).  They
   // win where the rays are fewer than the waves that fit (512 x 512 of 512^3
   // u16 456 against 530 us, of 64^3 94 against 107) and lose elsewhere
   // (1920 x 1080 of 512^3 u16 770 against 660, of 128^3 259 against 237).

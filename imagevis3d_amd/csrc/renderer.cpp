@@ -1665,8 +1665,8 @@ static int fill_job_table(JobTable* t, const RaycastParams* jobs, int n, const L
   }
   // Gradient launches look their TFs up through vector memory, which they
   // are bound by; the jobs' distinct 2D TF masks (8 KiB at 256 x 256) or
-  // small 1D TFs go to LDS as far as they fit.  32 KiB leave room for the
-  // three 4-wave work-groups per CU that the registers allow.
+  // small 1D TFs go to LDS as far as they fit the 32 KiB that such a launch
+  // reserves.
   t->h.n_tables = 0;
   if (li.mode == 1 || li.lighting) {
     int used = 0;  // 16-byte units

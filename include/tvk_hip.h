@@ -441,10 +441,10 @@ int tvk_set_kernel_tuning(tvk_renderer* r, uint32_t samples_per_batch, uint32_t 
 /* Waves per work-group (4 or 8; default 4) of the raycast variants that do
  * not stage the 1D TF in LDS (2D TF, lighting without LDS TF, isosurface,
  * MIP, mixed-TF launches); no counterpart in the reference, chosen by the
- * autotuner (TVK_TUNE_LAUNCH).  Those variants fit 2-3 waves per SIMD, so
- * 4-wave work-groups put up to 12 waves on a CU and 8-wave ones 8: more
- * waves hide more latency on cache-friendly volumes and thrash the caches
- * on very large ones.  The image does not depend on it. */
+ * autotuner (TVK_TUNE_LAUNCH).  Those variants fit 2-6 waves per SIMD
+ * (trilinear 2-5); where that is an odd number 4-wave work-groups put more
+ * waves on a CU than 8-wave ones: more waves hide more latency on
+ * cache-friendly volumes and thrash the caches on very large ones.  The image does not depend on it. */
 int tvk_set_work_group_waves(tvk_renderer* r, uint32_t waves);
 /* LDS staging of the 1D march (no counterpart in the reference; chosen by
  * the autotuner, TVK_TUNE_LAUNCH): with on = 1, 1D-TF launches without
