@@ -92,7 +92,7 @@ int main() {
     printf("OK frame\n");
   }
   for (int up = 0; up < 2; ++up) {  // someone who needs the workers gets them after the pieces at hand
-    const std::vector<unsigned char> src = pattern(320 * MiB, 11);
+    const std::vector<unsigned char> src = pattern(160 * MiB, 11);
     std::vector<unsigned char> dst(src.size());
     g_copied = 0;
     size_t asked = 0, got = 0;
