@@ -245,12 +245,16 @@ hipError_t HostPipe::Download(int device, const CopyPiece* pieces, size_t n, hip
     const hipError_t q = c < ahead ? hipSuccess : fetch(c, t);
     return q == hipSuccess ? drain(c, t) : q;
   };
+  bool queued = false;  // copies that nobody has waited for
   auto plain = [&](size_t c, size_t t) {
+    if (c < ahead) return drain(c, t);
     const CopyPiece p = cut(c);
-    return c < ahead ? drain(c, t) : hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+    queued = true;
+    return hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
   };
   if (e == hipSuccess) e = all_pieces(device, m, piece, plain);
-  const hipError_t last = hipStreamSynchronize(stream);  // the copies made without the workers, or an error's
+  if (e == hipSuccess && !queued) return e;  // every piece has been drained
+  const hipError_t last = hipStreamSynchronize(stream);
   return e == hipSuccess ? last : e;
 }
 
