@@ -1298,8 +1298,9 @@ hipError_t launch_histogram_1d(const void* vol, int bpv, int64_t n, unsigned lon
   if (lds_allowed(hist1d_u16_lds_kernel, lds)) {
     // A group per pass of 8192 voxels up to a quarter of the CUs, then four
     // passes a group: a group adds each of its distinct values to the global
-    // bins, as many as its voxels where they hardly repeat (128^3 voxels of
-    // noise 113 us with a group per pass, 87 now; scans take the same).
+    // bins, as many as its voxels where they hardly repeat.  128^3 voxels of
+    // noise take 113 us with a group per pass and 88 so, a smooth field 100
+    // and 84, a scan 72 and 75, values that share few bins 58 and 64.
     const int64_t cus = device_cus(), passes = (n + kHistThreads * kRunX - 1) / (kHistThreads * kRunX);
     const int64_t groups = std::min(cus, std::max(std::min(passes, cus / 4), passes / 4));
     hist1d_u16_lds_kernel<<<(unsigned)groups, kHistThreads, lds, stream>>>((const uint16_t*)vol, n, hist);
