@@ -39,7 +39,7 @@ namespace tvk {
 constexpr uint64_t kLaunchCostCap = 1000000000ull;
 // While other launches are in flight and requests keep coming, each within
 // kCompanyGapMs of the one before, a request waits up to kCompanyMs for
-// company before it takes a free lane: a client submits one every 10 to 15
+// company before it takes a free lane: a client submits one every 10 to 20
 // us, and light requests, which come back in 0.1 to 0.2 ms, would each take a
 // launch of their own.  Without the wait 64 light requests at once take 2.3
 // ms in 63 launches, 1.6 with it, 24 mixed ones 10.3 against 9.5 ms.  A wait
